@@ -185,11 +185,12 @@ int mmoe_gfull_stack(int L0, int nl);
 #define MMOE_R_HN 19      /* float [nb][2048] work input */
 int mmoe_read(int what, void *dst, size_t bytes);
 int mmoe_set_debug(int on);
-/* Batches of <= 8 tokens use three fused decode kernels (default on); off = the grouped-GEMM path. */
+/* One token uses three fused decode kernels, two and three tokens their down kernel (default on); off = the grouped
+ * path of larger batches. */
 int mmoe_set_decode_path(int on);
-/* Batches whose pairs are tiled by 16 (fewer than 2048 pairs, above the decode path): 1 (default) = one fused
- * kernel per tile (gate/up, SiLU*up, act quantisation and down; the act never leaves the chip), 0 = the three
- * separate kernels. Both give identical results. */
+/* Batches whose pairs are tiled by 16 (fewer than 2048 pairs, above the decode path): 1 (default) = the fused kernels
+ * (few experts: gate/up and down with the act quantisation, each expert over many workgroups; else one kernel per
+ * tile), 0 = the three separate kernels. All give identical results. */
 int mmoe_set_expert_path(int fused);
 /* Router of batches of >= 512 tokens in batch order: 0 (default) = bf16 MFMA logits on the input split into
  * three exact bf16 parts, with every expert that a rounding bound cannot exclude from a token's top 8 recomputed

@@ -936,17 +936,34 @@ __global__ void __launch_bounds__(512) k_group(const int *__restrict__ hist, int
     }
 }
 
-// Host-given grouping (gpre_moe / gfull_moe / gpux): plan from ustart; one thread.
-__global__ void k_plan_from_ustart(const int *__restrict__ ustart, int nu, Plan *__restrict__ plan, int tn, Tile *__restrict__ tiles) {
-    if (threadIdx.x != 0) return;
-    int t = 0;
-    for (int u = 0; u < nu; u++) {
-        int c = ustart[u + 1] - ustart[u];
-        plan->ue[u] = u; plan->ustart[u] = ustart[u]; plan->tstart[u] = t;
-        for (int i = 0; i * tn < c; i++) tiles[t++] = Tile{u, ustart[u] + i * tn, min(tn, c - i * tn), 0};
+// One tile of the split down kernel (split.h): its pairs and its expert's pointers
+struct DnTile { int p0, n, pad0, pad1; const uint8_t *dc; const float *ds; };
+// Host-given grouping (gpre_moe / gfull_moe / gpux): plan, tile table and (dt given) the split path's tile records from
+// ustart. Thread = used expert; the tile offsets are a scan over them (one thread walking the experts took 28 us for a
+// 128-token chunk's 250).
+__global__ void __launch_bounds__(256) k_plan_from_ustart(const int *__restrict__ ustart, int nu, Plan *__restrict__ plan, int tn,
+                                                          Tile *__restrict__ tiles, const ExpPtr *__restrict__ eptr, DnTile *__restrict__ dt) {
+    __shared__ int wt[4];
+    int t = threadIdx.x, l = t & 63, wv = t >> 6;
+    int p0 = t < nu ? ustart[t] : 0, c = t < nu ? ustart[t + 1] - p0 : 0, nt = (c + tn - 1) / tn, ist = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) { int a = __shfl_up(ist, o, 64); if (l >= o) ist += a; }
+    if (l == 63) wt[wv] = ist;
+    __syncthreads();
+    for (int k = 0; k < wv; k++) ist += wt[k];
+    int t0 = ist - nt;
+    if (t < nu) {
+        plan->ue[t] = t; plan->ustart[t] = p0; plan->tstart[t] = t0;
+        for (int i = 0; i < nt; i++) {
+            int n = min(tn, c - i * tn);
+            tiles[t0 + i] = Tile{t, p0 + i * tn, n, 0};
+            if (dt) dt[t0 + i] = DnTile{p0 + i * tn, n, 0, 0, eptr[t].dc, eptr[t].ds};
+        }
+        if (t == nu - 1) {
+            plan->ustart[nu] = p0 + c; plan->tstart[nu] = ist;
+            plan->nu = nu; plan->np = p0 + c; plan->ntile_gu = ist; plan->tn = tn;
+        }
     }
-    plan->ustart[nu] = ustart[nu]; plan->tstart[nu] = t;
-    plan->nu = nu; plan->np = ustart[nu]; plan->ntile_gu = t; plan->tn = tn;
 }
 
 // rint of four values |v| <= 2^22 as four int8 in one word (byte i = value i), and their sum added to *sum.

@@ -20,6 +20,7 @@
 #include <vector>
 #include "kernels.h"
 #include "decode.h"
+#include "split.h"
 #include "attn.h"
 #ifndef GU16_W
 #define GU16_W 4    // small-tile gate/up: waves per workgroup, 16-row fragments per wave
@@ -69,6 +70,7 @@ struct Work {
     int *qsumx = nullptr, *qsuma = nullptr;
     int *dbg_gu = nullptr, *dbg_dn = nullptr;
     int *dov = nullptr;             // the same for the int16 down results
+    DnTile *dt = nullptr;           // tile records of the split down kernel [SP_MAXP]
     int *eu = nullptr, *pu = nullptr;   // expert -> used-expert index [256], pair -> used-expert index [P]
     bool compact = false;           // the last expert stage left down as int16 (k_combine16)
     int hist_used = 0;              // entries of hist the device grouping filled; the combine clears them
@@ -160,7 +162,7 @@ static int work_alloc(Work &w, int maxtok, Carve *c = nullptr) {
         wbuf(w.utok, P * 4, c) || wbuf(w.uw, P * 4, c) || wbuf(w.tp, P * 4, c) || wbuf(w.sp, P * 4, c) ||
         wbuf(w.ustart, (MNE + 1) * 4, c) || wbuf(w.qx, T * MH, c) || wbuf(w.qsx, T * 4, c) || wbuf(w.qsumx, T * 4, c) ||
         wbuf(w.act, P * MFF * 4, c) || wbuf(w.qa, P * MFF, c) || wbuf(w.qsa, P * 4, c) || wbuf(w.qsuma, P * 4, c) ||
-        wbuf(w.down, P * MH * 4, c) || wbuf(w.eu, MNE * 4, c) || wbuf(w.pu, P * 4, c) || wbuf(w.rcnt, T * 4, c))
+        wbuf(w.down, P * MH * 4, c) || wbuf(w.eu, MNE * 4, c) || wbuf(w.pu, P * 4, c) || wbuf(w.rcnt, T * 4, c) || wbuf(w.dt, sizeof(DnTile) * SP_MAXP, c))
         return -1;
     // the per-chunk expert counts start at zero; the combine after k_group clears what it used
     kl(k_fill_zero, (nch * MNE + 255) / 256, 256, 0, w.hist, nch * MNE);
@@ -363,6 +365,29 @@ static int launch_expert16(Work &w, int maxtiles, int *dg, int *dd, bool grp) {
     return launch(MMOE_K_GATEUP, [&] { kl(k_expert16<E16_W, E16_RING, 0, E16_GL>, grid8(maxtiles), 64 * E16_W, 0, w.plan, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx,
                                           w.down, dg ? w.act : nullptr, w.qa, w.qsa, w.qsuma, dg, dd, GroupIn{}); });
 }
+// Tiles of 16 with few used experts: every expert over many workgroups (split.h) instead of one (k_expert16). Per layer,
+// split gate/up + down against k_expert16: 5 tokens 14.9 us / 35.0, 23 tokens 31.0 / 37.5, 32 tokens 36.4 / 38.6; with
+// the workgroups that find no tile of their own, 40 tokens 40.8 / 39.3. Host groupings know their tiles (none is empty):
+// 163 tiles 32.6 / 36.8, 222 tiles 40.9 / 40.8.
+#define SP_MAXTILE 192
+static bool split_use(int np, int ntile, bool grp) { return grp ? np <= SP_MAXP : ntile > 0 && ntile <= SP_MAXTILE; }
+template <int KS>
+static int launch_gu_split(Work &w, int items, int *dg, bool grp) {
+    if (grp) {
+        SplitGroup g{w.top, w.tw, w.grp_nb, w.grp_tab, w.plan, w.tiles, w.eptr, w.eu, w.utok, w.uw, w.tp, w.sp, w.pu, w.dt};
+        return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, true>, (items + 1) * 8 * KS, 256, 0, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, g); });
+    }
+    return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, false>, items * 8 * KS, 256, 0, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, SplitGroup{}); });
+}
+// items: pairs (grp: a pair may turn out to start a tile) or tiles. The columns of a row over 4, 2 or 1 waves: 16 pairs
+// 6.2 / 6.6 / 8.2 us, 24 pairs 7.5 / 7.7 / 8.4, 40 pairs 10.9 / 9.3 / 11.1, 64 pairs 14.3 / 12.4 / 12.0
+static int launch_split_gateup(Work &w, int items, int *dg, bool grp) {
+    return items <= 24 ? launch_gu_split<4>(w, items, dg, grp) : items <= 48 ? launch_gu_split<2>(w, items, dg, grp) : launch_gu_split<1>(w, items, dg, grp);
+}
+static int launch_split(Work &w, int items, int *dg, int *dd, bool grp) {
+    if (launch_split_gateup(w, items, dg, grp)) return -1;
+    return launch(MMOE_K_DOWN, [&] { kl(k_dn_split, items * 16, 256, 0, w.dt, w.act, w.qa, w.qsa, w.qsuma, w.down, dd); });
+}
 static int launch_quant_act(Work &w, int maxtiles, int tn, int np, int *dg) {
     if (tn == 64) {
         // checks on: activation from the int32 sums in the debug buffer; else gate/up wrote it already
@@ -373,11 +398,13 @@ static int launch_quant_act(Work &w, int maxtiles, int tn, int np, int *dg) {
 }
 // device_grouping: the grouping came from k_group (pu is valid), so the 64-token-tile path may
 // hand the down results to k_combine as int16 (not with checks on: the tests read them as fp32)
-static int stage_experts(Work &w, int np, int nu_max, int tn, bool device_grouping) {
+static int stage_experts(Work &w, int np, int nu_max, int tn, bool device_grouping, int ntile = 0) {
     int maxtiles = np / tn + (nu_max < np ? nu_max : np);
     int *dg = S.debug ? w.dbg_gu : nullptr, *dd = S.debug ? w.dbg_dn : nullptr;
     w.compact = device_grouping && tn == 64 && !S.debug;
-    if (tn == 16 && S_expert16) return launch_expert16(w, maxtiles, dg, dd, device_grouping && w.grp16);
+    const bool grp = device_grouping && w.grp16;
+    if (tn == 16 && S_expert16 && split_use(np, ntile, grp)) return launch_split(w, grp ? np : ntile, dg, dd, grp);
+    if (tn == 16 && S_expert16) return launch_expert16(w, maxtiles, dg, dd, grp);
     if (launch_gateup(w, maxtiles, tn, dg)) return -1;
     if (!w.compact && launch_quant_act(w, maxtiles, tn, np, dg)) return -1;
     if (launch_down(w, maxtiles, tn, dd, w.compact)) return -1;
@@ -394,45 +421,44 @@ static int stage_combine(Work &w, int nb, float *d_x, int mode) {
     return launch(MMOE_K_COMBINE, [&] { kl(k_combine, (n + 255) / 256, 256, 0, w.down, w.uw, w.tp, w.sp, w.tw, nb, d_x, mode, hz, hzn); });
 }
 
-// Small batches (decode): three kernels, see decode.h. in = hn (do_norm 0) or the hidden state x whose
-// rmsnorm(post_ln) is the MoE input (do_norm 1); hn is also written to w.hn.
-static bool S_dec_enabled = true;
-static int launch_dec_gateup(Work &w, int nb, int L) {
-    int maxu = nb * MTOPK < MNE ? nb * MTOPK : MNE;
-    int *dg = S.debug ? w.dbg_gu : nullptr;
-    const ExpPtr *tab = S.layers[L].tab;
-    return launch(MMOE_K_GATEUP, [&] { kl(k_dec_gateup, dim3(MFF / 8, maxu), 256, 0, w.rl, w.hn, nb, tab, w.top, w.tw, w.plan, w.utok, w.uw, w.tp, w.sp, w.eptr, w.qx, w.qsx, w.qsumx, w.act, dg); });
-}
 static int launch_dec_down(Work &w, int nb, float *d_x, int order) {
     int *dd = S.debug ? w.dbg_dn : nullptr;
     int mode = order == MMOE_ORDER_STEP ? MMOE_COMBINE_STEP : MMOE_COMBINE_BATCH;
     return launch(MMOE_K_DOWN, [&] { kl(k_dec_down, MH / 8, 256, 0, w.plan, w.eptr, w.act, w.qa, w.qsa, w.qsuma, w.tp, w.sp, w.uw, w.tw, nb, d_x, mode, w.down, dd); });
 }
-static int moe_dec(Work &w, int L, const float *in, int do_norm, int nb, float *d_x, int order) {
+// One token (decode): three kernels, see decode.h. in = hn (do_norm 0) or the hidden state x whose
+// rmsnorm(post_ln) is the MoE input (do_norm 1); hn is also written to w.hn.
+static bool S_dec_enabled = true;
+static int moe_dec(Work &w, int L, const float *in, int do_norm, float *d_x, int order) {
     LayerW &lw = S.layers[L];
     const uint16_t *pln = do_norm ? lw.post_ln : nullptr;
+    int *dg = S.debug ? w.dbg_gu : nullptr;
+    const ExpPtr *tab = lw.tab;
     w.rl_nb = 0;
     if (order == MMOE_ORDER_STEP) {
-        if (launch(MMOE_K_ROUTER, [&] { kl(k_dec_route<16>, MNE * 16 / 64, 64, 0, in, nb, pln, do_norm, lw.rc16, lw.bias, w.hn, w.rl); })) return -1;
+        if (launch(MMOE_K_ROUTER, [&] { kl(k_dec_route<16>, MNE * 16 / 64, 64, 0, in, pln, do_norm, lw.rc16, lw.bias, w.hn, w.rl); })) return -1;
     } else {
-        if (launch(MMOE_K_ROUTER, [&] { kl(k_dec_route<8>, MNE * 8 / 64, 64, 0, in, nb, pln, do_norm, lw.rc8, lw.bias, w.hn, w.rl); })) return -1;
+        if (launch(MMOE_K_ROUTER, [&] { kl(k_dec_route<8>, MNE * 8 / 64, 64, 0, in, pln, do_norm, lw.rc8, lw.bias, w.hn, w.rl); })) return -1;
     }
-    w.rl_nb = nb;
-    if (launch_dec_gateup(w, nb, L)) return -1;
-    return launch_dec_down(w, nb, d_x, order);
+    w.rl_nb = 1;
+    if (launch(MMOE_K_GATEUP, [&] { kl(k_dec_gateup, dim3(MFF / 8, MTOPK), 256, 0, w.rl, w.hn, tab, w.top, w.tw, w.plan, w.utok, w.uw, w.tp, w.sp, w.eptr, w.qx, w.qsx, w.qsumx, w.act, dg); })) return -1;
+    return launch_dec_down(w, 1, d_x, order);
 }
 
 // Whole MoE layer on device buffers: x[b] += MoE_L(hn[b]), with the work set w (no allocation here)
 static int moe_dev(Work &w, int L, const float *d_hn, int nb, float *d_x, int order) {
     if (nb < 1 || nb > w.maxtok) { seterr("nb %d outside 1..%d (mmoe_init)", nb, w.maxtok); return -1; }
     if (L < 0 || L >= NLMAX || !S.layers[L].tab) { seterr("layer %d not set (mmoe_set_layer)", L); return -1; }
-    if (nb <= DEC_MAXTOK && S_dec_enabled) return moe_dec(w, L, d_hn, 0, nb, d_x, order);
+    if (nb == 1 && S_dec_enabled) return moe_dec(w, L, d_hn, 0, d_x, order);
     int np = nb * MTOPK, tn = tile_tn(np);
     // below 512 tokens the router launch also runs the top-8 and the quantisation; the per-chunk counts are for
     // k_group, which the fused small-tile kernel does without (it groups itself)
     bool grp16 = tn == 16 && S_expert16 && nb <= E16_GRP_MAXTOK;
     if (stage_router(w, L, d_hn, nb, order, false, S_router_tk, grp16 ? nullptr : w.hist)) return -1;
     int rc = stage_route_group(w, L, nb, tn, d_hn);
+    // two or three tokens: the decode down kernel, which also combines (decode.h)
+    if (!rc && nb <= DEC_MAXTOK && S_dec_enabled && w.grp16)
+        return launch_split_gateup(w, np, S.debug ? w.dbg_gu : nullptr, true) ? -1 : launch_dec_down(w, nb, d_x, order);
     if (!rc) rc = stage_experts(w, np, MNE, tn, true);
     if (!rc) rc = stage_combine(w, nb, d_x, order == MMOE_ORDER_STEP ? MMOE_COMBINE_STEP : MMOE_COMBINE_BATCH);
     if (rc && w.hist_used) {   // a stage failed before the combine cleared the expert counts: clear them here
@@ -454,15 +480,16 @@ static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, 
     for (int u = 0; u < nu; u++) if (ustart[u + 1] < ustart[u]) { seterr("ustart not ascending at %d", u); return -1; }
     for (int a = 0; a < np; a++) if (ptok[a] < 0 || ptok[a] >= nb) { seterr("ptok[%d] = %d outside 0..%d", a, ptok[a], nb - 1); return -1; }
     if (tp) for (int i = 0; i < nb * MTOPK; i++) if (tp[i] < 0 || tp[i] >= np) { seterr("tp[%d] = %d outside 0..%d", i, tp[i], np - 1); return -1; }
-    int tn = tile_tn(np);
+    int tn = tile_tn(np), ntile = 0;
+    for (int u = 0; u < nu; u++) ntile += (ustart[u + 1] - ustart[u] + tn - 1) / tn;
     HC(hipMemcpyAsync(w.eptr, eptr_h, sizeof(ExpPtr) * nu, hipMemcpyHostToDevice, S.st));
     HC(hipMemcpyAsync(w.ustart, ustart, sizeof(int) * (nu + 1), hipMemcpyHostToDevice, S.st));
     HC(hipMemcpyAsync(w.utok, ptok, sizeof(int) * np, hipMemcpyHostToDevice, S.st));
     if (pw) HC(hipMemcpyAsync(w.uw, pw, sizeof(float) * np, hipMemcpyHostToDevice, S.st));
     if (tp) HC(hipMemcpyAsync(w.tp, tp, sizeof(int) * nb * MTOPK, hipMemcpyHostToDevice, S.st));
-    if (launch(MMOE_K_GROUP, [&] { kl(k_plan_from_ustart, 1, 64, 0, w.ustart, nu, w.plan, tn, w.tiles); })) return -1;
+    if (launch(MMOE_K_GROUP, [&] { kl(k_plan_from_ustart, 1, 256, 0, w.ustart, nu, w.plan, tn, w.tiles, w.eptr, ntile <= SP_MAXTILE ? w.dt : (DnTile *)nullptr); })) return -1;
     if (stage_quant_x(w, w.hn, nb)) return -1;
-    return stage_experts(w, np, nu, tn, false);
+    return stage_experts(w, np, nu, tn, false, ntile);
 }
 
 // loc (maple.c:276-277: per used expert 6 x (region slot, byte offset)) + regs -> device pointers
@@ -894,7 +921,7 @@ int mmoe_init(int maxtok) {
     return work_debug(S.main, S.debug);
 }
 
-// Small batches take the three-kernel decode path unless switched off (tests compare both paths).
+// One token takes the three-kernel decode path, two and three its down kernel, unless switched off (tests compare).
 // Every setter below changes what a captured graph holds (kernels, pointers it passes): each drops the graph
 // before the change, so the next mmoe_stack_graph captures again and no replay touches freed memory.
 int mmoe_set_router_mode(int exact) { if (mmoe_graph_reset()) return -1; S_router_exact = exact != 0; return 0; }
@@ -1030,7 +1057,7 @@ int mmoe_stack_dev(int L0, int nl, float *d_x, int nb, int order) {
     if (!w.maxtok || nb < 1 || nb > w.maxtok) { seterr("mmoe_stack_dev: nb %d outside capacity %d", nb, w.maxtok); return -1; }
     for (int L = L0; L < L0 + nl; L++) {
         if (L < 0 || L >= NLMAX || !S.layers[L].tab) { seterr("mmoe_stack_dev: layer %d not set", L); return -1; }
-        if (nb <= DEC_MAXTOK && S_dec_enabled) { if (moe_dec(w, L, d_x, 1, nb, d_x, order)) return -1; continue; }
+        if (nb == 1 && S_dec_enabled) { if (moe_dec(w, L, d_x, 1, d_x, order)) return -1; continue; }
         const uint16_t *pw = S.layers[L].post_ln;
         if (order == MMOE_ORDER_STEP || nb < 512) {   // the chain router forms hn itself (no rmsnorm launch)
             w.norm_x = d_x; w.norm_w = pw;
