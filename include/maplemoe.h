@@ -224,7 +224,7 @@ void *mmoe_stream(void);
 #define MMOE_K_QKN 10           /* k_qkn: head norms, rope, fp16 cache */
 #define MMOE_K_ATT_SCORES 11
 #define MMOE_K_ATT_SOFTMAX 12
-#define MMOE_K_ATT_PV 13
+#define MMOE_K_ATT_PV 13        /* weighted sum of values; with short windows the whole attention (k_att_local) */
 #define MMOE_PROF_NKERNELS 14
 int mmoe_event_record(int slot);
 double mmoe_event_elapsed_ms(void);

@@ -708,13 +708,13 @@ static int set_router(int L, const uint16_t *router);
 // gfull_attn runs rmsnorm -> q/k/v (k_dense) -> q/k norm + rope + fp16 cache -> attention -> o (x += o) ->
 // post-norm -> router logits (exact chains), and gfull_moe the experts of the pairs the host picked.
 // One sequence; the chunk's nb tokens sit at positions pos0 .. pos0+nb-1 of a cache of ctx positions.
-#define AT_SC_NB 2    // tokens per k_att_scores workgroup
 #define GF_NWL 4352   // per layer in the norms gfull_init receives: in_ln 2048 | post_ln 2048 | q_norm 128 | k_norm 128
 static struct {
-    int ready, ctx, win, maxtok, pos0;
+    int ready, ctx, win, maxtok, pos0, sst;   // sst: ctx in whole blocks of 16 (score rows, caches)
     uint16_t *nw;                 // bf16 [24][4352] (the fp32 norms are bf16 values: exact)
     float *cs;                    // [ctx][32][2]
-    __half *kc, *vc, *ko;         // [24][ctx][512] x 2, [24][maxtok][1024]
+    __half *kc; float *vc;        // [24][4 heads][sst][128] each: the fp16 cache values, v widened (attn.h)
+    __half *ko;                   // [24][maxtok][1024]
     uint16_t *ko_host;            // gfull_read's copy
     float *qkv, *att, *sc, *inv, *mx;  // [maxtok][3072], [maxtok][2048], [maxtok * 16][ctx], [maxtok * 16] x 2
     double t_attn;
@@ -736,13 +736,14 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     for (size_t i = 0; i < nw.size(); i++) { uint32_t u; memcpy(&u, &norms[i], 4); nw[i] = (uint16_t)(u >> 16); }
     HC(hipMalloc(&GF.nw, nw.size() * 2)); HC(hipMemcpy(GF.nw, nw.data(), nw.size() * 2, hipMemcpyHostToDevice));
     HC(hipMalloc(&GF.cs, (size_t)ctx * 64 * 4)); HC(hipMemcpy(GF.cs, cs, (size_t)ctx * 64 * 4, hipMemcpyHostToDevice));
-    size_t kvb = (size_t)24 * ctx * 512 * 2, kob = (size_t)24 * maxtok * 1024 * 2;
-    HC(hipMalloc(&GF.kc, kvb)); HC(hipMalloc(&GF.vc, kvb)); HC(hipMalloc(&GF.ko, kob));
-    HC(hipMemset(GF.kc, 0, kvb)); HC(hipMemset(GF.vc, 0, kvb));
+    GF.sst = (ctx + 15) & ~15;
+    size_t kvb = (size_t)24 * GF.sst * 512 * 2, kob = (size_t)24 * maxtok * 1024 * 2;
+    HC(hipMalloc(&GF.kc, kvb)); HC(hipMalloc(&GF.vc, 2 * kvb)); HC(hipMalloc(&GF.ko, kob));
+    HC(hipMemset(GF.kc, 0, kvb)); HC(hipMemset(GF.vc, 0, 2 * kvb));
     GF.ko_host = (uint16_t *)malloc(kob);
     if (!GF.ko_host) { seterr("gfull_init: %zu bytes of host memory", kob); return -1; }
     HC(hipMalloc(&GF.qkv, (size_t)maxtok * 3072 * 4)); HC(hipMalloc(&GF.att, (size_t)maxtok * MH * 4));
-    HC(hipMalloc(&GF.sc, (size_t)maxtok * 16 * ctx * 4)); HC(hipMalloc(&GF.inv, (size_t)maxtok * 16 * 4)); HC(hipMalloc(&GF.mx, (size_t)maxtok * 16 * 4));
+    HC(hipMalloc(&GF.sc, (size_t)maxtok * 16 * GF.sst * 4)); HC(hipMalloc(&GF.inv, (size_t)maxtok * 16 * 4)); HC(hipMalloc(&GF.mx, (size_t)maxtok * 16 * 4));
     for (int L = 0; L < 24; L++) {
         if (set_router(L, router + (size_t)L * MNE * MH)) return -1;
         LayerW &lw = S.layers[L];
@@ -751,7 +752,7 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     }
     GF.ctx = ctx; GF.win = win; GF.maxtok = maxtok; GF.ready = 1;
     S.gfull = true;
-    fprintf(stderr, "maplemoe: whole layers on the card, key/value cache %.0f MB\n", 2.0 * kvb / 1e6);
+    fprintf(stderr, "maplemoe: whole layers on the card, key/value cache %.0f MB\n", 3.0 * kvb / 1e6);
     return 0;
 }
 // a new chunk: nb hidden vectors (embeddings) at positions pos0..
@@ -771,26 +772,34 @@ static int gfull_attn_launch(int L, int glob) {
         seterr("gfull_attn: layer %d projections are not q,k,v (3072 rows) and o (2048) (gpre_dense_add)", L); return -1;
     }
     Work &w = S.main;
-    int nb = S.gfull_nb, pos0 = GF.pos0, ctx = GF.ctx, win = GF.win, g = 2 * L;
+    int nb = S.gfull_nb, pos0 = GF.pos0, sst = GF.sst, win = GF.win, g = 2 * L;
     const uint16_t *nwl = GF.nw + (size_t)L * GF_NWL;
-    __half *kcl = GF.kc + (size_t)L * ctx * 512, *vcl = GF.vc + (size_t)L * ctx * 512, *kol = GF.ko + (size_t)L * GF.maxtok * 1024;
+    __half *kcl = GF.kc + (size_t)L * sst * 512;
+    float *vcl = GF.vc + (size_t)L * sst * 512;
+    __half *kol = GF.ko + (size_t)L * GF.maxtok * 1024;
     if (launch(MMOE_K_RMSNORM, [&] { kl(k_rmsnorm, nb, 256, 0, w.x, nwl, w.hn, nb); })) return -1;
     if (stage_quant_x(w, w.hn, nb)) return -1;
     if (launch(MMOE_K_DENSE, [&] {
         kl(k_dense<DENSE_W>, dim3(3072 / (64 * DENSE_W), (nb + 63) / 64), 64 * DENSE_W, 0, DN.dmat + g * 3, DN.drbs + g * 4, DN.n[g], nb, 3072, w.qx, w.qsx, w.qsumx, GF.qkv);
     })) return -1;
     if (launch(MMOE_K_QKN, [&] {
-        kl(k_qkn, nb, 256, 0, GF.qkv, pos0, glob, nwl + 4096, nwl + 4224, GF.cs, kcl, vcl, kol, GF.mx);
+        kl(k_qkn, nb, 256, 0, GF.qkv, pos0, glob, nwl + 4096, nwl + 4224, GF.cs, kcl, vcl, kol, GF.mx, sst);
     })) return -1;
-    int span = glob ? pos0 + nb : std::min(pos0 + nb, win + AT_SC_NB);   // positions one token group can see
-    if (launch(MMOE_K_ATT_SCORES, [&] {
-        kl(k_att_scores<AT_SC_NB>, dim3((nb + AT_SC_NB - 1) / AT_SC_NB * 4, (span + 63) / 64), 64, 0, GF.qkv, nb, pos0, glob, win, kcl, GF.sc, GF.mx, ctx);
-    })) return -1;
-    if (launch(MMOE_K_ATT_SOFTMAX, [&] { kl(k_att_softmax, nb, 256, 0, pos0, glob, win, GF.sc, GF.mx, GF.inv, ctx); })) return -1;
-    if (launch(MMOE_K_ATT_PV, [&] {   // small chunks: fewer tokens per workgroup, more workgroups
-        if (nb > 256) kl(k_att_pv<4>, (nb + 3) / 4 * 4, 256, 0, nb, pos0, glob, win, GF.sc, GF.mx, GF.inv, vcl, GF.att, ctx);
-        else kl(k_att_pv<2>, (nb + 1) / 2 * 4, 256, 0, nb, pos0, glob, win, GF.sc, GF.mx, GF.inv, vcl, GF.att, ctx);
-    })) return -1;
+    // blocks of 16 positions that a row tile's windows can overlap
+    int tiles = (nb + AT_G - 1) / AT_G * 4, span = glob ? pos0 + nb : std::min(pos0 + nb, win + AT_G), blocks = (span + 15) / 16 + 1;
+    if (blocks * 16 <= AT_LOCAL_T) {
+        int ldt = (blocks + 1) / 2 * 32 + 4;
+        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_local, tiles, 256, (size_t)16 * ldt * 4, GF.qkv, nb, pos0, glob, win, kcl, vcl, GF.att, ldt, sst); })) return -1;
+    } else {
+        // one run of k_att_scores takes a tile's whole window, unless the tiles alone are fewer than 1024 workgroups (then
+        // runs of at least 8 blocks)
+        int split = std::max(1, std::min((1024 + tiles - 1) / tiles, blocks / 8)), run = (blocks + 4 * split - 1) / (4 * split) * 4;
+        if (launch(MMOE_K_ATT_SCORES, [&] {
+            kl(k_att_scores, dim3(tiles, (blocks + run - 1) / run), 256, 0, GF.qkv, nb, pos0, glob, win, kcl, GF.sc, GF.mx, sst, run);
+        })) return -1;
+        if (launch(MMOE_K_ATT_SOFTMAX, [&] { kl(k_att_softmax, nb, 256, 0, pos0, glob, win, GF.sc, GF.mx, GF.inv, sst); })) return -1;
+        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_pv, tiles, 256, 0, nb, pos0, glob, win, GF.sc, GF.mx, GF.inv, vcl, GF.att, sst); })) return -1;
+    }
     if (stage_quant_x(w, GF.att, nb)) return -1;
     return launch(MMOE_K_DENSE, [&] {
         kl(k_dense<DENSE_W, true>, dim3(MH / (64 * DENSE_W), (nb + 63) / 64), 64 * DENSE_W, 0, DN.dmat + (g + 1) * 3, DN.drbs + (g + 1) * 4, DN.n[g + 1], nb, MH, w.qx, w.qsx, w.qsumx, w.x);
