@@ -48,6 +48,8 @@ struct Plan {
 };
 // One token tile of a grouped launch: used expert, first pair, pairs in the tile (<= TN)
 struct Tile { int u, p0, n, pad; };
+// One tile of the split down kernel (split.h): its pairs and its expert's pointers
+struct DnTile { int p0, n, pad0, pad1; const uint8_t *dc; const float *ds; };
 
 __device__ __forceinline__ float bf16f(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 
@@ -936,36 +938,6 @@ __global__ void __launch_bounds__(512) k_group(const int *__restrict__ hist, int
     }
 }
 
-// One tile of the split down kernel (split.h): its pairs and its expert's pointers
-struct DnTile { int p0, n, pad0, pad1; const uint8_t *dc; const float *ds; };
-// Host-given grouping (gpre_moe / gfull_moe / gpux): plan, tile table and (dt given) the split path's tile records from
-// ustart. Thread = used expert; the tile offsets are a scan over them (one thread walking the experts took 28 us for a
-// 128-token chunk's 250).
-__global__ void __launch_bounds__(256) k_plan_from_ustart(const int *__restrict__ ustart, int nu, Plan *__restrict__ plan, int tn,
-                                                          Tile *__restrict__ tiles, const ExpPtr *__restrict__ eptr, DnTile *__restrict__ dt) {
-    __shared__ int wt[4];
-    int t = threadIdx.x, l = t & 63, wv = t >> 6;
-    int p0 = t < nu ? ustart[t] : 0, c = t < nu ? ustart[t + 1] - p0 : 0, nt = (c + tn - 1) / tn, ist = nt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { int a = __shfl_up(ist, o, 64); if (l >= o) ist += a; }
-    if (l == 63) wt[wv] = ist;
-    __syncthreads();
-    for (int k = 0; k < wv; k++) ist += wt[k];
-    int t0 = ist - nt;
-    if (t < nu) {
-        plan->ue[t] = t; plan->ustart[t] = p0; plan->tstart[t] = t0;
-        for (int i = 0; i < nt; i++) {
-            int n = min(tn, c - i * tn);
-            tiles[t0 + i] = Tile{t, p0 + i * tn, n, 0};
-            if (dt) dt[t0 + i] = DnTile{p0 + i * tn, n, 0, 0, eptr[t].dc, eptr[t].ds};
-        }
-        if (t == nu - 1) {
-            plan->ustart[nu] = p0 + c; plan->tstart[nu] = ist;
-            plan->nu = nu; plan->np = p0 + c; plan->ntile_gu = ist; plan->tn = tn;
-        }
-    }
-}
-
 // rint of four values |v| <= 2^22 as four int8 in one word (byte i = value i), and their sum added to *sum.
 // v + 1.5 * 2^23 lies in [2^23, 2^24), where the float spacing is 1, so the addition rounds v to the nearest
 // integer, ties to even (rintf's rounding), and the low byte of the sum's bit pattern is that integer mod 256.
@@ -1034,6 +1006,72 @@ __global__ void __launch_bounds__(256) k_quant(const float *__restrict__ x, int 
     int row = blockIdx.x * 4 + wv;
     if (row >= nrows) return;
     quant_wave<N>(x + (size_t)row * N, l, q + (size_t)row * N, qs + row, qsum + row);
+}
+
+// A host-given grouping (gpre_moe / gfull_moe / gpux) taken over in one launch: block 0 forms the plan, the tile table and
+// (dt given) the split path's tile records from ustart, blocks 1 .. ncopy copy the used experts' pointers and the pair
+// tables into device memory, the others quantise the nb input rows (maple.c prep), 4 a block. The tables (and the input
+// of a few rows) are read where the host put them, in pinned memory: five copies of a few KB took longer than the
+// expert kernels of a decode call. In block 0 thread = used expert; the tile offsets are a scan over them (one thread
+// walking the experts took 28 us for a 128-token chunk's 250).
+struct HostGroup { const ExpPtr *ep; const int *ustart, *ptok; const float *pw; const int *tp; int nu, np, ntp; };
+__global__ void __launch_bounds__(256) k_host_group(HostGroup h, int ncopy, Plan *__restrict__ plan, int tn, Tile *__restrict__ tiles,
+                                                    DnTile *__restrict__ dt, ExpPtr *__restrict__ eptr, int *__restrict__ utok,
+                                                    float *__restrict__ uw, int *__restrict__ tp, const float *__restrict__ x, int nb,
+                                                    int8_t *__restrict__ qx, float *__restrict__ qsx, int *__restrict__ qsumx) {
+    __shared__ int wt[4];
+    int t = threadIdx.x, l = t & 63, wv = t >> 6;
+    if ((int)blockIdx.x > ncopy) {
+        int row = ((int)blockIdx.x - 1 - ncopy) * 4 + wv;
+        if (row < nb) quant_wave<MH>(x + (size_t)row * MH, l, qx + (size_t)row * MH, qsx + row, qsumx + row);
+        return;
+    }
+    if (blockIdx.x) {   // words: the pointers, then ptok, pw, tp
+        const int ne = h.nu * (int)(sizeof(ExpPtr) / 4), nw = h.pw ? h.np : 0, n = ne + h.np + nw + h.ntp;
+        for (int i = ((int)blockIdx.x - 1) * 256 + t; i < n; i += ncopy * 256) {
+            int k = i;
+            if (k < ne) { ((int *)eptr)[k] = ((const int *)h.ep)[k]; continue; }
+            if ((k -= ne) < h.np) { utok[k] = h.ptok[k]; continue; }
+            if ((k -= h.np) < nw) { uw[k] = h.pw[k]; continue; }
+            tp[k - nw] = h.tp[k - nw];
+        }
+        return;
+    }
+    int nu = h.nu, p0 = t < nu ? h.ustart[t] : 0, c = t < nu ? h.ustart[t + 1] - p0 : 0, nt = (c + tn - 1) / tn, ist = nt;
+    const uint8_t *dc = nullptr; const float *ds = nullptr;
+    if (dt && t < nu) { dc = h.ep[t].dc; ds = h.ep[t].ds; }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) { int a = __shfl_up(ist, o, 64); if (l >= o) ist += a; }
+    if (l == 63) wt[wv] = ist;
+    __syncthreads();
+    for (int k = 0; k < wv; k++) ist += wt[k];
+    int t0 = ist - nt;
+    if (t < nu) {
+        plan->ue[t] = t; plan->ustart[t] = p0; plan->tstart[t] = t0;
+        for (int i = 0; i < nt; i++) {
+            int n = min(tn, c - i * tn);
+            tiles[t0 + i] = Tile{t, p0 + i * tn, n, 0};
+            if (dt) dt[t0 + i] = DnTile{p0 + i * tn, n, 0, 0, dc, ds};
+        }
+        if (t == nu - 1) {
+            plan->ustart[nu] = p0 + c; plan->tstart[nu] = ist;
+            plan->nu = nu; plan->np = p0 + c; plan->ntile_gu = ist; plan->tn = tn;
+        }
+    }
+}
+
+// The routing results of nb tokens (mmoe_route) into one run of pinned host memory, [nu, ue 256, ustart 257] then top, tw,
+// utok, uw, tp of P words each; also clears the per-chunk expert counts for the next call.
+#define RO_HEAD 514
+__global__ void __launch_bounds__(256) k_route_out(const Plan *__restrict__ plan, const int *__restrict__ top, const int *__restrict__ tw,
+                                                   const int *__restrict__ utok, const int *__restrict__ uw, const int *__restrict__ tp,
+                                                   int P, int *__restrict__ out, int *__restrict__ hist, int nh) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < RO_HEAD + 5 * P; i += gridDim.x * 256) {
+        if (i < RO_HEAD) { out[i] = i == 0 ? plan->nu : i <= 256 ? plan->ue[i - 1] : plan->ustart[i - 257]; continue; }
+        int k = (i - RO_HEAD) / P, j = (i - RO_HEAD) % P;
+        out[i] = k == 0 ? top[j] : k == 1 ? tw[j] : k == 2 ? utok[j] : k == 3 ? uw[j] : tp[j];
+    }
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < nh; i += gridDim.x * 256) hist[i] = 0;
 }
 
 __global__ void __launch_bounds__(256) k_topk_quant(const float *__restrict__ rl, const float *__restrict__ hn, int nb,

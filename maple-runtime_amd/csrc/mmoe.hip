@@ -105,8 +105,20 @@ __global__ void k_fill_zero(int *p, int n) { int i = blockIdx.x * 256 + threadId
 struct Region { const void *host; size_t len; uint8_t *dev; };
 struct LayerW { ExpPtr *tab = nullptr; uint16_t *router = nullptr; uint16_t *rc16 = nullptr, *rc8 = nullptr; float *rf8 = nullptr, *w1max = nullptr; uint16_t *post_ln = nullptr; float *bias = nullptr; };
 
+// Pinned host memory that kernels read and write in place (coherent): tables from the host in a ring of blocks, each reused
+// only after the launch that reads it has run, and one block for results. Sized for the largest grouping (2048 tokens).
+#define HS_RING 4
+#define HS_X (64 << 10)   // an input of up to 8 rows travels with its tables
+#define HS_TABLES (MNE * sizeof(ExpPtr) + (MNE + 1 + 3) * 4 + 3 * (size_t)MMOE_MAXTOK * MTOPK * 4 + HS_X)
+#define HS_OUT ((RO_HEAD + 5 * (size_t)MMOE_MAXTOK * MTOPK) * 4)
+struct HostRing { uint8_t *p = nullptr; hipEvent_t ev = nullptr; bool used = false; };
+
 static struct {
     bool ready = false;
+    HostRing hs[HS_RING]; int hs_next = 0;
+    uint8_t *hs_out = nullptr;
+    hipEvent_t te[2] = {};     // device seconds of the synchronous calls
+    hipStream_t cst = nullptr; // copies to the host beside the compute stream
     ExpPtr *zero_tab = nullptr;     // mmoe_route: the expert table k_group reads when no layer is involved
     hipStream_t st = nullptr;
     Work main;                 // gpre / gfull / mmoe
@@ -119,7 +131,7 @@ static struct {
     double t_region = 0.0;     // seconds spent copying regions into HBM
     // gpux
     int gx_layers = 0, gx_slots = 0; uint8_t *gx_mem = nullptr;
-    hipEvent_t gx_ev = nullptr; int gx_np = 0;
+    hipEvent_t gx_ev = nullptr; int gx_np = 0; uint8_t *gx_out = nullptr;   // gx_out: pinned, the call's outputs
     // gfull
     bool gfull = false; int gfull_nb = 0;
     double t_moe = 0.0;
@@ -198,7 +210,11 @@ static int ctx_ready() {
     if (hipGetDeviceCount(&n) != hipSuccess || n < 1) { seterr("no HIP device"); return -1; }
     HC(hipStreamCreateWithFlags(&S.st, hipStreamNonBlocking));
     HC(hipEventCreate(&S.pe[0])); HC(hipEventCreate(&S.pe[1]));
-    HC(hipEventCreate(&S.gx_ev));
+    HC(hipEventCreate(&S.te[0])); HC(hipEventCreate(&S.te[1]));
+    HC(hipEventCreateWithFlags(&S.gx_ev, hipEventDisableTiming));
+    HC(hipStreamCreateWithFlags(&S.cst, hipStreamNonBlocking));
+    for (HostRing &r : S.hs) { HC(hipHostMalloc((void **)&r.p, HS_TABLES)); HC(hipEventCreateWithFlags(&r.ev, hipEventDisableTiming)); }
+    HC(hipHostMalloc((void **)&S.hs_out, HS_OUT));
     int dev = 0; HC(hipGetDevice(&dev));
     HC(hipDeviceGetAttribute(&S.ncu, hipDeviceAttributeMultiprocessorCount, dev));
     // the no-alloc work set: carved from the static scratch of this device (one device per process here)
@@ -471,9 +487,9 @@ static int moe_dev(Work &w, int L, const float *d_hn, int nb, float *d_x, int or
 }
 
 // Experts for a host-given grouping (gpre_moe, gfull_moe, gpux): ustart[nu+1], ptok, pw, tp on the host,
-// eptr[nu] resolved on the host. Input activations in w.hn.
+// eptr[nu] resolved on the host. Input activations in w.hn, or x_h on the host.
 static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, const int *ustart, const int *ptok,
-                                 const float *pw, const int *tp) {
+                                 const float *pw, const int *tp, const float *x_h = nullptr) {
     if (nu < 1 || nu > MNE) { seterr("nu %d outside 1..256", nu); return -1; }
     int np = ustart[nu];
     if (nb < 1 || nb > w.maxtok || np < 1 || np > w.maxp) { seterr("nb %d / pairs %d exceed capacity %d / %d", nb, np, w.maxtok, w.maxp); return -1; }
@@ -482,13 +498,27 @@ static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, 
     if (tp) for (int i = 0; i < nb * MTOPK; i++) if (tp[i] < 0 || tp[i] >= np) { seterr("tp[%d] = %d outside 0..%d", i, tp[i], np - 1); return -1; }
     int tn = tile_tn(np), ntile = 0;
     for (int u = 0; u < nu; u++) ntile += (ustart[u + 1] - ustart[u] + tn - 1) / tn;
-    HC(hipMemcpyAsync(w.eptr, eptr_h, sizeof(ExpPtr) * nu, hipMemcpyHostToDevice, S.st));
-    HC(hipMemcpyAsync(w.ustart, ustart, sizeof(int) * (nu + 1), hipMemcpyHostToDevice, S.st));
-    HC(hipMemcpyAsync(w.utok, ptok, sizeof(int) * np, hipMemcpyHostToDevice, S.st));
-    if (pw) HC(hipMemcpyAsync(w.uw, pw, sizeof(float) * np, hipMemcpyHostToDevice, S.st));
-    if (tp) HC(hipMemcpyAsync(w.tp, tp, sizeof(int) * nb * MTOPK, hipMemcpyHostToDevice, S.st));
-    if (launch(MMOE_K_GROUP, [&] { kl(k_plan_from_ustart, 1, 256, 0, w.ustart, nu, w.plan, tn, w.tiles, w.eptr, ntile <= SP_MAXTILE ? w.dt : (DnTile *)nullptr); })) return -1;
-    if (stage_quant_x(w, w.hn, nb)) return -1;
+    HostRing &r = S.hs[S.hs_next];
+    S.hs_next = (S.hs_next + 1) % HS_RING;
+    if (r.used) HC(hipEventSynchronize(r.ev));
+    uint8_t *q = r.p;
+    auto put = [&](const void *src, size_t n) { void *d = q; memcpy(d, src, n); q += (n + 15) / 16 * 16; return d; };
+    HostGroup h{};
+    h.ep = (const ExpPtr *)put(eptr_h, sizeof(ExpPtr) * nu);
+    h.ustart = (const int *)put(ustart, sizeof(int) * (nu + 1));
+    h.ptok = (const int *)put(ptok, sizeof(int) * np);
+    if (pw) h.pw = (const float *)put(pw, sizeof(float) * np);
+    if (tp) h.tp = (const int *)put(tp, sizeof(int) * nb * MTOPK);
+    const float *x = w.hn;
+    size_t xb = (size_t)nb * MH * 4;
+    if (x_h && xb <= HS_X) x = (const float *)put(x_h, xb);
+    else if (x_h) HC(hipMemcpyAsync(w.hn, x_h, xb, hipMemcpyHostToDevice, S.st));
+    h.nu = nu; h.np = np; h.ntp = tp ? nb * MTOPK : 0;
+    int words = nu * (int)(sizeof(ExpPtr) / 4) + np + (pw ? np : 0) + h.ntp, ncopy = std::min((words + 1023) / 1024, 64);
+    if (launch(MMOE_K_GROUP, [&] { kl(k_host_group, 1 + ncopy + (nb + 3) / 4, 256, 0, h, ncopy, w.plan, tn, w.tiles, ntile <= SP_MAXTILE ? w.dt : (DnTile *)nullptr,
+                                      w.eptr, w.utok, w.uw, w.tp, x, nb, w.qx, w.qsx, w.qsumx); })) return -1;
+    HC(hipEventRecord(r.ev, S.st));
+    r.used = true;
     return stage_experts(w, np, nu, tn, false, ntile);
 }
 
@@ -564,19 +594,15 @@ double gpre_moe(const float *x, int nb, int nu, const uint32_t *loc, const int *
     if (nb < 1 || nb > w.maxtok) { seterr("gpre_moe: nb %d outside 1..%d", nb, w.maxtok); return -1.0; }
     ExpPtr ep[MNE];
     if (nu < 1 || nu > MNE || resolve_loc(loc, regs, nu, ep)) { if (nu < 1 || nu > MNE) seterr("gpre_moe: nu %d", nu); return -1.0; }
-    hipEvent_t a, b;
-    if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) { seterr("gpre_moe: event"); return -1.0; }
-    auto fail = [&] { (void)hipEventDestroy(a); (void)hipEventDestroy(b); return -1.0; };
+    hipEvent_t a = S.te[0], b = S.te[1];
     (void)hipEventRecord(a, S.st);
-    if (hipMemcpyAsync(w.hn, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st) != hipSuccess) { seterr("gpre_moe: copy x"); return fail(); }
-    if (experts_host_grouping(w, nb, nu, ep, ustart, ptok, pw, tp)) return fail();
-    if (stage_combine(w, nb, w.x, MMOE_COMBINE_OVERWRITE)) return fail();
+    if (experts_host_grouping(w, nb, nu, ep, ustart, ptok, pw, tp, x)) return -1.0;
+    if (stage_combine(w, nb, w.x, MMOE_COMBINE_OVERWRITE)) return -1.0;
     (void)hipEventRecord(b, S.st);
     if (hipMemcpyAsync(y, w.x, (size_t)nb * MH * 4, hipMemcpyDeviceToHost, S.st) != hipSuccess || hipStreamSynchronize(S.st) != hipSuccess) {
-        seterr("gpre_moe: %s", hipGetErrorString(hipGetLastError())); return fail();
+        seterr("gpre_moe: %s", hipGetErrorString(hipGetLastError())); return -1.0;
     }
     float ms = 0; (void)hipEventElapsedTime(&ms, a, b);
-    (void)hipEventDestroy(a); (void)hipEventDestroy(b);
     S.t_moe += ms * 1e-3;
     return ms * 1e-3;
 }
@@ -677,21 +703,18 @@ double gpre_dense(int g, const float *x, int nb, float *y) {
     if (nb < 1 || nb > DN.maxtok) { seterr("gpre_dense: nb %d outside 1..%d", nb, DN.maxtok); return -1.0; }
     Work &w = S.main;
     int ys = DN.rows[g], nrb = ys / (64 * DENSE_W);
-    hipEvent_t a, b;
-    if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) { seterr("gpre_dense: event"); return -1.0; }
-    auto fail = [&] { (void)hipEventDestroy(a); (void)hipEventDestroy(b); return -1.0; };
+    hipEvent_t a = S.te[0], b = S.te[1];
     (void)hipEventRecord(a, S.st);
-    if (hipMemcpyAsync(w.hn, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st) != hipSuccess) { seterr("gpre_dense: copy x"); return fail(); }
-    if (stage_quant_x(w, w.hn, nb)) return fail();
+    if (hipMemcpyAsync(w.hn, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st) != hipSuccess) { seterr("gpre_dense: copy x"); return -1.0; }
+    if (stage_quant_x(w, w.hn, nb)) return -1.0;
     if (launch(MMOE_K_DENSE, [&] {
             kl(k_dense<DENSE_W>, dim3(nrb, (nb + 63) / 64), 64 * DENSE_W, 0, DN.dmat + g * 3, DN.drbs + g * 4, DN.n[g], nb, ys, w.qx, w.qsx, w.qsumx, DN.y);
-        })) return fail();
+        })) return -1.0;
     (void)hipEventRecord(b, S.st);
     if (hipMemcpyAsync(y, DN.y, (size_t)nb * ys * 4, hipMemcpyDeviceToHost, S.st) != hipSuccess || hipStreamSynchronize(S.st) != hipSuccess) {
-        seterr("gpre_dense: %s", hipGetErrorString(hipGetLastError())); return fail();
+        seterr("gpre_dense: %s", hipGetErrorString(hipGetLastError())); return -1.0;
     }
     float ms = 0; (void)hipEventElapsedTime(&ms, a, b);
-    (void)hipEventDestroy(a); (void)hipEventDestroy(b);
     DN.t += ms * 1e-3;
     return ms * 1e-3;
 }
@@ -715,7 +738,10 @@ static struct {
     float *cs;                    // [ctx][32][2]
     __half *kc; float *vc;        // [24][4 heads][sst][128] each: the fp16 cache values, v widened (attn.h)
     __half *ko;                   // [24][maxtok][1024]
-    uint16_t *ko_host;            // gfull_read's copy
+    uint16_t *ko_host;            // gfull_read's copy (pinned)
+    hipEvent_t kev[24], cev;      // layer's keys and values written; copies so far done
+    uint32_t copied, busy;        // layers whose keys and values are on their way to ko_host (this chunk's; any chunk's)
+    bool want_ko, captured;       // the last gfull_read asked for them; a caller has captured mmoe_gfull_stack
     float *qkv, *att, *sc, *inv, *mx;  // [maxtok][3072], [maxtok][2048], [maxtok * 16][ctx], [maxtok * 16] x 2
     double t_attn;
 } GF;
@@ -731,7 +757,8 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     void **dbuf[] = {(void **)&GF.nw, (void **)&GF.cs, (void **)&GF.kc, (void **)&GF.vc, (void **)&GF.ko,
                      (void **)&GF.qkv, (void **)&GF.att, (void **)&GF.sc, (void **)&GF.inv, (void **)&GF.mx};
     for (void **pp : dbuf) if (*pp) { HC(hipFree(*pp)); *pp = nullptr; }
-    free(GF.ko_host); GF.ko_host = nullptr;
+    HC(hipStreamSynchronize(S.cst));
+    if (GF.ko_host) { HC(hipHostFree(GF.ko_host)); GF.ko_host = nullptr; }
     std::vector<uint16_t> nw((size_t)24 * GF_NWL);
     for (size_t i = 0; i < nw.size(); i++) { uint32_t u; memcpy(&u, &norms[i], 4); nw[i] = (uint16_t)(u >> 16); }
     HC(hipMalloc(&GF.nw, nw.size() * 2)); HC(hipMemcpy(GF.nw, nw.data(), nw.size() * 2, hipMemcpyHostToDevice));
@@ -740,8 +767,12 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     size_t kvb = (size_t)24 * GF.sst * 512 * 2, kob = (size_t)24 * maxtok * 1024 * 2;
     HC(hipMalloc(&GF.kc, kvb)); HC(hipMalloc(&GF.vc, 2 * kvb)); HC(hipMalloc(&GF.ko, kob));
     HC(hipMemset(GF.kc, 0, kvb)); HC(hipMemset(GF.vc, 0, 2 * kvb));
-    GF.ko_host = (uint16_t *)malloc(kob);
-    if (!GF.ko_host) { seterr("gfull_init: %zu bytes of host memory", kob); return -1; }
+    HC(hipHostMalloc((void **)&GF.ko_host, kob));
+    if (!GF.cev) {
+        HC(hipEventCreateWithFlags(&GF.cev, hipEventDisableTiming));
+        for (hipEvent_t &e : GF.kev) HC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    GF.copied = GF.busy = 0; GF.want_ko = true; GF.captured = false;
     HC(hipMalloc(&GF.qkv, (size_t)maxtok * 3072 * 4)); HC(hipMalloc(&GF.att, (size_t)maxtok * MH * 4));
     HC(hipMalloc(&GF.sc, (size_t)maxtok * 16 * GF.sst * 4)); HC(hipMalloc(&GF.inv, (size_t)maxtok * 16 * 4)); HC(hipMalloc(&GF.mx, (size_t)maxtok * 16 * 4));
     for (int L = 0; L < 24; L++) {
@@ -760,7 +791,7 @@ void gfull_begin(const float *x, int nb, int pos0) {
     S.gfull_nb = 0;   // a rejected chunk leaves no chunk: gfull_attn / gfull_moe then report it
     if (!S.gfull || nb < 1 || nb > S.main.maxtok) { seterr("gfull_begin: not set up or nb %d out of range", nb); return; }
     if (GF.ready && (nb > GF.maxtok || pos0 < 0 || pos0 + nb > GF.ctx)) { seterr("gfull_begin: positions %d..%d past ctx %d", pos0, pos0 + nb - 1, GF.ctx); return; }
-    S.gfull_nb = nb; GF.pos0 = pos0;
+    S.gfull_nb = nb; GF.pos0 = pos0; GF.copied = 0;
     HCV(hipMemcpyAsync(S.main.x, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st));
 }
 // The attention half of layer L (asynchronous): x += o(attention(q, k, v of rmsnorm(x, in_ln))), k and v into
@@ -770,6 +801,10 @@ static int gfull_attn_launch(int L, int glob) {
     if (L < 0 || L >= 24) { seterr("gfull_attn: layer %d", L); return -1; }
     if (DN.rows[2 * L] != 3072 || DN.rows[2 * L + 1] != 2048) {
         seterr("gfull_attn: layer %d projections are not q,k,v (3072 rows) and o (2048) (gpre_dense_add)", L); return -1;
+    }
+    if (GF.busy >> L & 1) {   // a copy of the layer's last keys and values may still be reading them
+        HC(hipStreamWaitEvent(S.st, GF.cev, 0));
+        GF.copied &= ~(1u << L); GF.busy &= ~(1u << L);
     }
     Work &w = S.main;
     int nb = S.gfull_nb, pos0 = GF.pos0, sst = GF.sst, win = GF.win, g = 2 * L;
@@ -807,8 +842,8 @@ static int gfull_attn_launch(int L, int glob) {
 }
 // The attention half of layer L and the router: rl gets nb x 256 logits. Synchronous; returns device seconds.
 double gfull_attn(int L, int glob, float *rl) {
-    hipEvent_t a, b;
-    if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) { seterr("gfull_attn: event"); return -1.0; }
+    if (ctx_ready()) return -1.0;
+    hipEvent_t a = S.te[0], b = S.te[1];
     (void)hipEventRecord(a, S.st);
     int rc = gfull_attn_launch(L, glob);
     (void)hipEventRecord(b, S.st);
@@ -816,7 +851,6 @@ double gfull_attn(int L, int glob, float *rl) {
     if (!rc && hipStreamSynchronize(S.st) != hipSuccess) { seterr("gfull_attn: stream"); rc = -1; }
     float ms = 0;
     if (!rc) (void)hipEventElapsedTime(&ms, a, b);
-    (void)hipEventDestroy(a); (void)hipEventDestroy(b);
     if (rc) return -1.0;
     GF.t_attn += ms * 1e-3;
     return ms * 1e-3;
@@ -839,10 +873,17 @@ void gfull_read(float *x, const uint16_t **ko) {
         *ko = NULL;
         if (GF.ready) {   // the chunk's nb rows of every layer only (the [24][maxtok][1024] layout is kept)
             size_t pitch = (size_t)GF.maxtok * 1024 * 2, rows = (size_t)(S.gfull_nb ? S.gfull_nb : GF.maxtok) * 1024 * 2;
-            HCV(hipMemcpy2D(GF.ko_host, pitch, GF.ko, pitch, rows, 24, hipMemcpyDeviceToHost));
+            HCV(hipStreamSynchronize(S.cst));
+            for (int L = 0, n; L < 24; L += n) {   // runs of layers that mmoe_gfull_stack has not copied beside its work
+                bool have = GF.copied >> L & 1;
+                for (n = 1; L + n < 24 && (GF.copied >> (L + n) & 1) == have; n++) {}
+                if (!have) HCV(hipMemcpy2D((char *)GF.ko_host + L * pitch, pitch, (char *)GF.ko + L * pitch, pitch, rows, n, hipMemcpyDeviceToHost));
+            }
+            GF.copied = GF.busy = 0;
             *ko = GF.ko_host;
         }
     }
+    GF.want_ko = ko != nullptr;
 }
 void gfull_write_x(const float *x) {
     if (!S.gfull) { seterr("gfull_write_x: not set up"); return; }
@@ -857,6 +898,7 @@ int gpux_init(int layers, int slots) {
     if (ctx_ready()) return -1;
     if (layers < 1 || layers > NLMAX || slots < 1 || slots > 256) { seterr("gpux_init: layers %d / slots %d out of range", layers, slots); return -1; }
     if (!S.dec.maxtok && work_alloc(S.dec, MMOE_GPUX_MAXTOK)) return -1;
+    if (!S.gx_out) HC(hipHostMalloc((void **)&S.gx_out, (size_t)S.dec.maxp * MH * 4));
     if (work_debug(S.dec, S.debug)) return -1;
     if (S.gx_mem) {   // a second set-up replaces the first (its slots are gone until uploaded again)
         uint8_t *old = S.gx_mem;
@@ -892,8 +934,9 @@ static void *gpux_start(int L, const float *x, int nb, int nu, const int *slots,
         if (slots[k] < 0 || slots[k] >= S.gx_slots) { seterr("gpux: slot %d out of range", slots[k]); return NULL; }
         ep[k] = slot_ptr(L, slots[k]);
     }
-    HCN(hipMemcpyAsync(w.hn, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st));
-    if (experts_host_grouping(w, nb, nu, ep, pstart, ptok, NULL, NULL)) return NULL;
+    S.gx_np = 0;
+    if (experts_host_grouping(w, nb, nu, ep, pstart, ptok, NULL, NULL, x)) return NULL;
+    HCN(hipMemcpyAsync(S.gx_out, w.down, (size_t)pstart[nu] * MH * 4, hipMemcpyDeviceToHost, S.st));   // beside the caller's own work
     HCN(hipEventRecord(S.gx_ev, S.st));
     S.gx_np = pstart[nu];
     return (void *)&S.gx_ev;
@@ -901,8 +944,8 @@ static void *gpux_start(int L, const float *x, int nb, int nu, const int *slots,
 static void gpux_finish(void *h, float *out, int np) {
     if (h != (void *)&S.gx_ev) { seterr("gpux_end: unknown handle"); return; }
     if (np != S.gx_np) { seterr("gpux_end: %d outputs asked, %d computed", np, S.gx_np); return; }
-    HCV(hipMemcpyAsync(out, S.dec.down, (size_t)np * MH * 4, hipMemcpyDeviceToHost, S.st));
-    HCV(hipStreamSynchronize(S.st));
+    HCV(hipEventSynchronize(S.gx_ev));
+    memcpy(out, S.gx_out, (size_t)np * MH * 4);
 }
 // n hits of one token: outputs out[k][2048] = down of slot k's expert (unweighted), maple.c:628-642
 void *gpux_begin(int L, const float *x, int n, const int *slots) {
@@ -1032,20 +1075,20 @@ int mmoe_route(const float *rl, int nb, int *top, float *tw, int *ue, int *ustar
         return -1;
     int rc = launch(MMOE_K_GROUP, [&] { kl(k_group, nch, 512, 0, w.hist, nb, w.plan, S.zero_tab, w.eptr, 64, w.tiles, w.eu, w.top, w.tw, w.utok,
                                            w.uw, w.tp, w.sp, w.pu); });
-    kl(k_fill_zero, (nch * MNE + 255) / 256, 256, 0, w.hist, nch * MNE);   // the per-chunk counts, for the next call
-    if (rc) { (void)hipGetLastError(); return -1; }
-    HC(hipGetLastError());
-    Plan pl;   // pageable: the copy completes before the synchronisation below returns
-    HC(hipMemcpyAsync(&pl, w.plan, sizeof(Plan), hipMemcpyDeviceToHost, S.st));
-    if (top) HC(hipMemcpyAsync(top, w.top, (size_t)P * 4, hipMemcpyDeviceToHost, S.st));
-    if (tw) HC(hipMemcpyAsync(tw, w.tw, (size_t)P * 4, hipMemcpyDeviceToHost, S.st));
-    if (utok) HC(hipMemcpyAsync(utok, w.utok, (size_t)P * 4, hipMemcpyDeviceToHost, S.st));
-    if (uw) HC(hipMemcpyAsync(uw, w.uw, (size_t)P * 4, hipMemcpyDeviceToHost, S.st));
-    if (tp) HC(hipMemcpyAsync(tp, w.tp, (size_t)P * 4, hipMemcpyDeviceToHost, S.st));
+    if (rc) {
+        kl(k_fill_zero, (nch * MNE + 255) / 256, 256, 0, w.hist, nch * MNE);   // the per-chunk counts, for the next call
+        (void)hipGetLastError();
+        return -1;
+    }
+    int *o = (int *)S.hs_out;   // results through one kernel into pinned memory (six copies to pageable memory: 0.1 ms)
+    if (launch(MMOE_K_GROUP, [&] { kl(k_route_out, std::min((RO_HEAD + 5 * P + 255) / 256, 256), 256, 0, w.plan, w.top, (const int *)w.tw, w.utok, (const int *)w.uw, w.tp,
+                                      P, o, w.hist, nch * MNE); })) return -1;
     HC(hipStreamSynchronize(S.st));
-    if (ue) memcpy(ue, pl.ue, sizeof(int) * pl.nu);
-    if (ustart) memcpy(ustart, pl.ustart, sizeof(int) * (pl.nu + 1));
-    return pl.nu;
+    void *dst[5] = {top, tw, utok, uw, tp};
+    for (int k = 0; k < 5; k++) if (dst[k]) memcpy(dst[k], o + RO_HEAD + k * P, (size_t)P * 4);
+    if (ue) memcpy(ue, o + 1, sizeof(int) * o[0]);
+    if (ustart) memcpy(ustart, o + 257, sizeof(int) * (o[0] + 1));
+    return o[0];
 }
 
 // mmoe_moe_dev for batches of up to MMOE_NOALLOC_MAXTOK tokens with every work buffer in the library's static
@@ -1081,13 +1124,32 @@ int mmoe_stack_dev(int L0, int nl, float *d_x, int nb, int order) {
     return 0;
 }
 
+// The layer's keys and values to the host on the copy stream, beside the layers that follow (for programs whose gfull_read
+// asks for them; a captured stack leaves them to gfull_read, also on its replays).
+static int ko_copy(int L) {
+    if (!GF.want_ko || GF.captured) return 0;
+    size_t pitch = (size_t)GF.maxtok * 1024 * 2;
+    HC(hipEventRecord(GF.kev[L], S.st));
+    HC(hipStreamWaitEvent(S.cst, GF.kev[L], 0));
+    HC(hipMemcpyAsync((char *)GF.ko_host + L * pitch, (char *)GF.ko + L * pitch, (size_t)S.gfull_nb * 1024 * 2, hipMemcpyDeviceToHost, S.cst));
+    HC(hipEventRecord(GF.cev, S.cst));
+    GF.copied |= 1u << L; GF.busy |= 1u << L;
+    return 0;
+}
+
 int mmoe_gfull_stack(int L0, int nl) {
     if (ctx_ready()) return -1;
     if (L0 < 0 || nl < 1 || L0 + nl > 24) { seterr("mmoe_gfull_stack: layers %d..%d outside 0..23", L0, L0 + nl - 1); return -1; }
     if (!GF.ready || !S.gfull_nb) { seterr("mmoe_gfull_stack: gfull_init / gfull_begin first"); return -1; }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(S.st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipStreamSynchronize(S.cst);
+        GF.captured = true; GF.copied = GF.busy = 0;
+    }
     for (int L = L0; L < L0 + nl; L++) {
         if (!S.layers[L].tab) { seterr("mmoe_gfull_stack: layer %d has no experts (mmoe_set_layer)", L); return -1; }
         if (gfull_attn_launch(L, (L % 4) == 3)) return -1;
+        if (ko_copy(L)) return -1;
         if (mmoe_stack_dev(L, 1, S.main.x, S.gfull_nb, MMOE_ORDER_BATCH)) return -1;
     }
     return 0;

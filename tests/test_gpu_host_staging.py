@@ -1,0 +1,97 @@
+"""Host data through the library's pinned blocks: gfull_moe calls queued one after the other (more than the ring of table
+blocks holds) against the same calls with a wait after each; and the keys and values that gfull_read hands out when
+mmoe_gfull_stack has copied them beside its work, against the ones gfull_read copies itself, over two chunks of
+different size, a chunk whose copies nobody read, a repeated stack and a partial one."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import maplemoe as M
+import pyoracle as O
+from helpers import SEED, HostLayer
+from test_gpu_attn import CTX, MAXTOK, gfull_model  # noqa: F401  (the fixture)
+
+pytestmark = pytest.mark.gpu
+H, NL = 2048, 4
+
+
+@pytest.fixture(scope="module")
+def model(gfull_model):  # noqa: F811
+    lib, _, post, routers, cs, norms, router_all = gfull_model
+    M.check(lib.gfull_init(CTX, MAXTOK, O.WIN, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init")
+    rids = []
+    for L in range(NL):
+        hl = HostLayer(SEED, L % 2)
+        rids.append(M.register_layer(L, hl.blk, routers[L % 2], post[L % 2]))
+    return lib, rids
+
+
+def test_queued_groupings(model):
+    lib, rids = model
+    rng = np.random.default_rng(SEED + 80)
+    nb, calls = 24, []
+    for k in range(10):
+        top = np.argsort(rng.random((nb, 256)), 1)[:, :8].astype(np.int32)
+        g = O.group(top, rng.random((nb, 8)).astype(np.float32))
+        calls.append((g, M.block_loc(0, list(g["ue"])), np.array([rids[k % NL], -1, -1, -1], np.int32), np.ascontiguousarray(g["tp"])))
+    x0 = rng.standard_normal((nb, H)).astype(np.float32)
+    out = []
+    for wait in (True, False):
+        lib.gfull_begin(M.ptr(x0), nb, 0)
+        assert lib.mmoe_gfull_post_norm(0, None) == 0    # the calls' input: hn of the chunk
+        for g, loc, regs, tp in calls:
+            lib.gfull_moe(g["nu"], M.ptr(loc), M.ptr(regs), M.ptr(g["ustart"]), M.ptr(g["utok"]), M.ptr(g["uw"]), M.ptr(tp))
+            if wait:
+                M.check(lib.mmoe_sync(), "sync")
+        x = np.empty((nb, H), np.float32)
+        lib.gfull_read(M.ptr(x), None)
+        out.append(x)
+    assert np.array_equal(out[0].view(np.int32), out[1].view(np.int32)) and not np.array_equal(out[0], x0)
+
+
+def read_kv(lib, nb):
+    p = C.c_void_p()
+    lib.gfull_read(None, C.addressof(p))
+    a = np.ctypeslib.as_array((C.c_uint16 * (24 * MAXTOK * 1024)).from_address(p.value)).reshape(24, MAXTOK, 1024)
+    return a[:NL, :nb].copy()
+
+
+def test_kv_copied_beside_the_stack(model):
+    lib, _ = model
+    rng = np.random.default_rng(SEED + 81)
+    chunks = [(0, 200), (200, 37), (237, 256)]
+    xs = [rng.standard_normal((nb, H)).astype(np.float32) for _, nb in chunks]
+
+    def run(read, stacks):
+        got = []
+        for (pos, nb), x in zip(chunks, xs):
+            lib.gfull_begin(M.ptr(x), nb, pos)
+            for L0, nl in stacks:
+                M.check(lib.mmoe_gfull_stack(L0, nl), "stack")
+            if read(nb):
+                got.append(read_kv(lib, nb))
+        return got
+
+    lib.gfull_read(None, None)                                   # not asked for: gfull_read copies it all
+    lib.gfull_begin(M.ptr(xs[0]), 200, 0)
+    want = []
+    for (pos, nb), x in zip(chunks, xs):
+        lib.gfull_begin(M.ptr(x), nb, pos)
+        M.check(lib.mmoe_gfull_stack(0, NL), "stack")
+        lib.gfull_read(None, None)
+        want.append(read_kv(lib, nb))
+        lib.gfull_read(None, None)
+    for name, read, stacks in (("beside", lambda nb: True, [(0, NL)]), ("unread chunk", lambda nb: nb != 37, [(0, NL)]),
+                               ("in parts", lambda nb: True, [(0, 1), (1, 3)])):
+        got = run(read, stacks)
+        ref = [w for w, (_, nb) in zip(want, chunks) if read(nb)]
+        assert all(np.array_equal(a, b) for a, b in zip(got, ref)), name
+    # the same chunk twice (the second stack starts from the first one's hidden state), read once
+    lib.gfull_begin(M.ptr(xs[0]), 200, 0)
+    M.check(lib.mmoe_gfull_stack(0, NL), "stack"); M.check(lib.mmoe_gfull_stack(0, NL), "stack")
+    twice = read_kv(lib, 200)
+    lib.gfull_read(None, None)
+    lib.gfull_begin(M.ptr(xs[0]), 200, 0)
+    M.check(lib.mmoe_gfull_stack(0, NL), "stack"); M.check(lib.mmoe_gfull_stack(0, NL), "stack")
+    assert np.array_equal(twice, read_kv(lib, 200)) and not np.array_equal(twice, want[0])
