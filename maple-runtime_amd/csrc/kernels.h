@@ -855,7 +855,7 @@ __global__ void __launch_bounds__(512) k_group(const int *__restrict__ hist, int
                                                const ExpPtr *__restrict__ layer_tab, ExpPtr *__restrict__ eptr_u, int tn,
                                                Tile *__restrict__ tiles, int *__restrict__ eu_out, const int *__restrict__ top,
                                                const float *__restrict__ tw, int *__restrict__ utok, float *__restrict__ uw,
-                                               int *__restrict__ tp, int *__restrict__ sp, int *__restrict__ pu) {
+                                               int *__restrict__ tp, int *__restrict__ sp, int *__restrict__ pu, DnTile *__restrict__ dt) {
     constexpr int MAXCH = (2048 + 63) / 64;
     __shared__ int sc[MNE], su[MNE], st[MNE], sbase[MNE], seu[MNE];
     __shared__ unsigned long long msk[MNE];
@@ -908,7 +908,11 @@ __global__ void __launch_bounds__(512) k_group(const int *__restrict__ hist, int
                 plan->ustart[uidx] = pstart;
                 plan->tstart[uidx] = tstart;
                 if (layer_tab) { v4i *d = (v4i *)(eptr_u + uidx); d[0] = lt0; d[1] = lt1; d[2] = lt2; }
-                for (int i = 0; i < nt; i++) tiles[tstart + i] = Tile{uidx, pstart + i * tn, min(tn, run - i * tn), 0};
+                for (int i = 0; i < nt; i++) {
+                    int n = min(tn, run - i * tn);
+                    tiles[tstart + i] = Tile{uidx, pstart + i * tn, n, 0};
+                    if (dt) { v4i *d = (v4i *)(dt + tstart + i); d[0] = v4i{pstart + i * tn, n, 0, 0}; d[1] = lt2; }   // lt2: dc, ds
+                }
             }
             if (e == MNE - 1) {
                 int nu = su[e];
@@ -1889,7 +1893,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_down(const Plan *__restrict__ pl
 // utok, uw, sp, pu and tp (a pair's rank among its token's 8 pairs is the number of the token's experts with a
 // smaller id, since pairs are ordered by expert); workgroup 0 writes the plan, tile table, expert pointers and
 // eu as k_group does. The outputs equal k_group's.
-#define E16_GRP_MAXTOK 256
+#define E16_GRP_MAXTOK 239   // 255 tokens: 86.8 us per layer (some CUs get a second tile) against 80 with k_group and the split kernels; 216: 68.7 / 76
 struct GroupIn { const int *top; const float *tw; int nb; const ExpPtr *layer_tab; Plan *plan; Tile *tiles; ExpPtr *eptr_u;
                  int *eu; int *utok; float *uw; int *tp; int *sp; int *pu; };
 template <int WAVES, int RING, int GRP = 0, int GL = 8>

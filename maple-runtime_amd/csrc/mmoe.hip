@@ -174,7 +174,7 @@ static int work_alloc(Work &w, int maxtok, Carve *c = nullptr) {
         wbuf(w.utok, P * 4, c) || wbuf(w.uw, P * 4, c) || wbuf(w.tp, P * 4, c) || wbuf(w.sp, P * 4, c) ||
         wbuf(w.ustart, (MNE + 1) * 4, c) || wbuf(w.qx, T * MH, c) || wbuf(w.qsx, T * 4, c) || wbuf(w.qsumx, T * 4, c) ||
         wbuf(w.act, P * MFF * 4, c) || wbuf(w.qa, P * MFF, c) || wbuf(w.qsa, P * 4, c) || wbuf(w.qsuma, P * 4, c) ||
-        wbuf(w.down, P * MH * 4, c) || wbuf(w.eu, MNE * 4, c) || wbuf(w.pu, P * 4, c) || wbuf(w.rcnt, T * 4, c) || wbuf(w.dt, sizeof(DnTile) * SP_MAXP, c))
+        wbuf(w.down, P * MH * 4, c) || wbuf(w.eu, MNE * 4, c) || wbuf(w.pu, P * 4, c) || wbuf(w.rcnt, T * 4, c) || wbuf(w.dt, sizeof(DnTile) * ((size_t)w.maxp / 16 + MNE + 8), c))
         return -1;
     // the per-chunk expert counts start at zero; the combine after k_group clears what it used
     kl(k_fill_zero, (nch * MNE + 255) / 256, 256, 0, w.hist, nch * MNE);
@@ -248,8 +248,12 @@ static int launch(int kid, F &&f) {
 // ------------------------------------------------------------------------------------------------------
 // Pipeline stages
 // ------------------------------------------------------------------------------------------------------
-static int tile_tn(int np) { return np >= 2048 ? 64 : 16; }
-static bool S_expert16 = true;   // tiles of 16: the fused whole-expert kernel (else three kernels)
+static bool S_expert16 = true;   // tiles of 16: the fused kernels (else three kernels)
+// Tiles of 16 up to 359 tokens: an expert then has few more than 16 pairs, and the split kernels (split.h) read its codes
+// about once, with more workgroups than the 64-pair tiles make. Whole layer, 16 / 64: balanced experts 300 tokens 84.5 /
+// 99.1 us, 400 tokens 95.5 / 102.7; with the Zipf bias (few experts of many tiles) 333 tokens 69.2 / 72.4, 511 tokens
+// 91.7 / 81.4: the line lies where the second would begin to lose.
+static int tile_tn(int np) { return np >= (S_expert16 ? 2880 : 2048) ? 64 : 16; }
 
 // Router logits of nb tokens (d_hn) with layer L's router; order 0 = batch (maple.c:853-889), 1 = step (bf_row)
 static bool S_router_exact = false;
@@ -333,7 +337,7 @@ static int stage_route_group(Work &w, int L, int nb, int tn, const float *d_hn) 
     w.hist_used = nch * MNE;   // cleared by this call's combine
     return launch(MMOE_K_GROUP, [&] {
         kl(k_group, nch, 512, 0, w.hist, nb, w.plan, S.layers[L].tab, w.eptr, tn, w.tiles, w.eu, w.top, w.tw, w.utok, w.uw,
-                                       w.tp, w.sp, w.pu);
+                                       w.tp, w.sp, w.pu, tn == 16 ? w.dt : (DnTile *)nullptr);
     });
 }
 
@@ -384,16 +388,16 @@ static int launch_expert16(Work &w, int maxtiles, int *dg, int *dd, bool grp) {
 // Tiles of 16 with few used experts: every expert over many workgroups (split.h) instead of one (k_expert16). Per layer,
 // split gate/up + down against k_expert16: 5 tokens 14.9 us / 35.0, 23 tokens 31.0 / 37.5, 32 tokens 36.4 / 38.6; with
 // the workgroups that find no tile of their own, 40 tokens 40.8 / 39.3. Host groupings know their tiles (none is empty):
-// 163 tiles 32.6 / 36.8, 222 tiles 40.9 / 40.8.
-#define SP_MAXTILE 192
-static bool split_use(int np, int ntile, bool grp) { return grp ? np <= SP_MAXP : ntile > 0 && ntile <= SP_MAXTILE; }
+// 163 tiles 32.6 / 36.8, 222 tiles 40.9 / 40.8, and past 256, when some CUs get a second tile, 275 tiles 51.4 / 65.7. With
+// the grouping from k_group (240 tokens and more; the host knows an upper bound of the tiles) always.
+static bool split_use(int np, int ntile, bool grp) { return grp ? np <= SP_MAXP : ntile <= 192 || ntile > 256; }
 template <int KS>
 static int launch_gu_split(Work &w, int items, int *dg, bool grp) {
     if (grp) {
         SplitGroup g{w.top, w.tw, w.grp_nb, w.grp_tab, w.plan, w.tiles, w.eptr, w.eu, w.utok, w.uw, w.tp, w.sp, w.pu, w.dt};
-        return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, true>, (items + 1) * 8 * KS, 256, 0, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, g); });
+        return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, true>, (items + 1) * 8 * KS, 256, 0, w.plan, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, g); });
     }
-    return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, false>, items * 8 * KS, 256, 0, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, SplitGroup{}); });
+    return launch(MMOE_K_GATEUP, [&] { kl(k_gu_split<KS, false>, items * 8 * KS, 256, 0, w.plan, w.tiles, w.eptr, w.utok, w.qx, w.qsx, w.qsumx, w.act, dg, SplitGroup{}); });
 }
 // items: pairs (grp: a pair may turn out to start a tile) or tiles. The columns of a row over 4, 2 or 1 waves: 16 pairs
 // 6.2 / 6.6 / 8.2 us, 24 pairs 7.5 / 7.7 / 8.4, 40 pairs 10.9 / 9.3 / 11.1, 64 pairs 14.3 / 12.4 / 12.0
@@ -402,7 +406,7 @@ static int launch_split_gateup(Work &w, int items, int *dg, bool grp) {
 }
 static int launch_split(Work &w, int items, int *dg, int *dd, bool grp) {
     if (launch_split_gateup(w, items, dg, grp)) return -1;
-    return launch(MMOE_K_DOWN, [&] { kl(k_dn_split, items * 16, 256, 0, w.dt, w.act, w.qa, w.qsa, w.qsuma, w.down, dd); });
+    return launch(MMOE_K_DOWN, [&] { kl(k_dn_split, items * 16, 256, 0, w.plan, w.dt, w.act, w.qa, w.qsa, w.qsuma, w.down, dd); });
 }
 static int launch_quant_act(Work &w, int maxtiles, int tn, int np, int *dg) {
     if (tn == 64) {
@@ -419,6 +423,7 @@ static int stage_experts(Work &w, int np, int nu_max, int tn, bool device_groupi
     int *dg = S.debug ? w.dbg_gu : nullptr, *dd = S.debug ? w.dbg_dn : nullptr;
     w.compact = device_grouping && tn == 64 && !S.debug;
     const bool grp = device_grouping && w.grp16;
+    if (device_grouping && !grp) ntile = maxtiles;
     if (tn == 16 && S_expert16 && split_use(np, ntile, grp)) return launch_split(w, grp ? np : ntile, dg, dd, grp);
     if (tn == 16 && S_expert16) return launch_expert16(w, maxtiles, dg, dd, grp);
     if (launch_gateup(w, maxtiles, tn, dg)) return -1;
@@ -515,7 +520,7 @@ static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, 
     else if (x_h) HC(hipMemcpyAsync(w.hn, x_h, xb, hipMemcpyHostToDevice, S.st));
     h.nu = nu; h.np = np; h.ntp = tp ? nb * MTOPK : 0;
     int words = nu * (int)(sizeof(ExpPtr) / 4) + np + (pw ? np : 0) + h.ntp, ncopy = std::min((words + 1023) / 1024, 64);
-    if (launch(MMOE_K_GROUP, [&] { kl(k_host_group, 1 + ncopy + (nb + 3) / 4, 256, 0, h, ncopy, w.plan, tn, w.tiles, ntile <= SP_MAXTILE ? w.dt : (DnTile *)nullptr,
+    if (launch(MMOE_K_GROUP, [&] { kl(k_host_group, 1 + ncopy + (nb + 3) / 4, 256, 0, h, ncopy, w.plan, tn, w.tiles, tn == 16 ? w.dt : (DnTile *)nullptr,
                                       w.eptr, w.utok, w.uw, w.tp, x, nb, w.qx, w.qsx, w.qsumx); })) return -1;
     HC(hipEventRecord(r.ev, S.st));
     r.used = true;
@@ -1074,7 +1079,7 @@ int mmoe_route(const float *rl, int nb, int *top, float *tw, int *ue, int *ustar
                                      (int8_t *)nullptr, (float *)nullptr, (int *)nullptr, w.hist); }))
         return -1;
     int rc = launch(MMOE_K_GROUP, [&] { kl(k_group, nch, 512, 0, w.hist, nb, w.plan, S.zero_tab, w.eptr, 64, w.tiles, w.eu, w.top, w.tw, w.utok,
-                                           w.uw, w.tp, w.sp, w.pu); });
+                                           w.uw, w.tp, w.sp, w.pu, (DnTile *)nullptr); });
     if (rc) {
         kl(k_fill_zero, (nch * MNE + 255) / 256, 256, 0, w.hist, nch * MNE);   // the per-chunk counts, for the next call
         (void)hipGetLastError();

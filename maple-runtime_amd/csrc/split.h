@@ -1,4 +1,4 @@
-// split.h -- gate/up and down of batches with few pairs (up to SP_MAXP), each expert spread over many workgroups.
+// split.h -- gate/up and down in tiles of 16 pairs, each expert spread over many workgroups.
 //
 // With few used experts, one workgroup per expert (k_expert16) leaves most CUs idle: a CU streams about 30 GB/s, so a
 // 798,720-byte expert takes 27 us however few there are. Here an expert's rows are split over 8 to 32 workgroups per
@@ -58,12 +58,10 @@ __device__ __forceinline__ void split_publish(const SplitGroup &g, void *lds) {
             g.dt[t0 + i] = DnTile{p0 + 16 * i, n, 0, 0, my.dc, my.ds};
         }
     }
-    int ntile = wt[0][2] + wt[1][2] + wt[2][2] + wt[3][2];
     if (t == MNE - 1) {
         g.plan->nu = isu; g.plan->np = isc; g.plan->ntile_gu = ist; g.plan->tn = 16;
         g.plan->ustart[isu] = isc; g.plan->tstart[isu] = ist;
     }
-    if (t >= ntile && t < P) g.dt[t] = DnTile{0, 0, 0, 0, nullptr, nullptr};   // the down grid has P tiles
     __syncthreads();
     if (e >= 0) {
         int before = popc64(msk[wv][e] & ((1ull << l) - 1ull)), lower = 0, b = t / MTOPK;
@@ -80,9 +78,9 @@ __device__ __forceinline__ void split_publish(const SplitGroup &g, void *lds) {
 // meet in LDS; used where the tiles alone would leave CUs idle). MFMA operands as k_gateup; the tile's n input rows in
 // LDS (the others hold whatever was there: their columns are never stored). act (fp32) to HBM.
 // GRP: tile = pair i's expert if i is its 1st, 17th, ... pair (else the workgroup leaves); block 0 publishes the
-// grouping. grid = (P + 1) 8 KS. !GRP: tile i of the plan; grid = ntile 8 KS.
+// grouping. grid = (P + 1) 8 KS. !GRP: tile i of the plan; grid = at least ntile 8 KS.
 template <int KS, bool GRP>
-__global__ void __launch_bounds__(256, 4) k_gu_split(const Tile *__restrict__ tiles, const ExpPtr *__restrict__ eptr,
+__global__ void __launch_bounds__(256, 4) k_gu_split(const Plan *__restrict__ plan, const Tile *__restrict__ tiles, const ExpPtr *__restrict__ eptr,
                                                   const int *__restrict__ utok, const int8_t *__restrict__ qx,
                                                   const float *__restrict__ qsx, const int *__restrict__ qsumx,
                                                   float *__restrict__ act, int *__restrict__ dbg, SplitGroup g) {
@@ -116,6 +114,7 @@ __global__ void __launch_bounds__(256, 4) k_gu_split(const Tile *__restrict__ ti
         for (int k = 0; k < SP_MAXP / 64; k++)
             if (tv[k] == e && rk[k] >= rank && rk[k] < rank + 16) toks[wv][rk[k] - rank] = (k * 64 + l) / MTOPK;
     } else {
+        if (item >= plan->ntile_gu) return;
         Tile tl = tiles[item];
         p0 = tl.p0; ntok = tl.n;
         ex = eptr[tl.u];
@@ -185,12 +184,13 @@ __global__ void __launch_bounds__(256, 4) k_gu_split(const Tile *__restrict__ ti
     }
 }
 
-// Down of one tile for 128 rows (wave w: RF = 2 fragments of 16): the tile's act is quantised in the workgroup while
+// Down of one tile for 64 RF rows (wave w: RF = 2 fragments of 16): the tile's act is quantised in the workgroup while
 // its codes are in flight (half-wave h takes pairs h, h + 8), D = (float)(sum - qsum) * qs * s_down[row] to HBM; the
-// tile's first workgroup also writes the int8 act out. grid = tiles x 16; a record with n = 0 is not a tile. One
-// fragment per wave (twice the workgroups, each quantising the tile again) takes 5.4 us against 5.6 us for 5 tokens and
-// 8.4 against 7.4 for 12, four fragments 6.3 and 8.0.
-__global__ void __launch_bounds__(256) k_dn_split(const DnTile *__restrict__ dt, const float *__restrict__ act,
+// tile's first workgroup also writes the int8 act out. grid = at least ntile x 16. One fragment per wave (twice the
+// workgroups, each quantising the tile again) takes 5.4 us against 5.6 us for 5 tokens and 8.4 against 7.4 for 12, four
+// fragments 6.3 and 8.0. Tiles of 32 pairs (two token fragments here and in k_gu_split, whose workgroups then fill the LDS
+// of a CU at two): 37.5 + 23.2 us at 300 tokens against 31.8 + 24.1.
+__global__ void __launch_bounds__(256) k_dn_split(const Plan *__restrict__ plan, const DnTile *__restrict__ dt, const float *__restrict__ act,
                                                   int8_t *__restrict__ qa, float *__restrict__ qsa, int *__restrict__ qsuma,
                                                   float *__restrict__ down, int *__restrict__ dbg) {
     constexpr int RF = 2, NSP = 32 / RF, GS = 128, QW = MFF + 16;
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(256) k_dn_split(const DnTile *__restrict__ dt,
     __shared__ int ss[16];
     int tid = threadIdx.x, l = tid & 63, G = l >> 4, r16 = l & 15, wv = tid >> 6;
     DnTile d = dt[blockIdx.x / NSP];
-    if (d.n == 0) return;
+    if ((int)(blockIdx.x / NSP) >= plan->ntile_gu) return;
     int part = blockIdx.x % NSP, row0 = (part * 4 + wv) * RF * 16, p0 = d.p0, ntok = d.n;
     const uint8_t *cp = d.dc + (uint32_t)(row0 + r16) * (MFF / 4) + (G >> 1) * 32 + (G & 1) * 16;
     // act before the codes: loads return in issue order and the quantisation is the longer chain

@@ -1,7 +1,8 @@
 """Gate/up and down of batches with few pairs, each expert spread over many workgroups (csrc/split.h), against k_group and
 the three separate kernels, bit for bit in every intermediate and in x, at the sizes where the dispatch changes: two and
 three tokens (the decode down kernel), 24 / 48 pairs (columns over 4, 2 or 1 waves), 256 pairs (the last batch whose pairs
-find their own tiles) and the one above it; host groupings of 1 to 193 tiles (192 is the last on the split kernels).
+find their own tiles) and the one above it; 240 to 359 tokens (tiles of 16 with the grouping of k_group) and the one above;
+host groupings of 1 to 193 tiles (192 is the last on the split kernels below 257) and of 257.
 The Zipf bias gives experts of more than 16 pairs, so further tiles of one expert occur."""
 import numpy as np
 import pytest
@@ -30,7 +31,7 @@ ITEMS = (("GU_I32", 1024, np.int32), ("ACT", 512, np.float32), ("QA", 512, np.in
 
 
 @pytest.mark.parametrize("zipf", [0, 1])
-@pytest.mark.parametrize("nb,order", [(2, 0), (3, 0), (3, 1), (4, 0), (6, 0), (7, 0), (20, 1), (31, 0), (32, 0), (33, 0)])
+@pytest.mark.parametrize("nb,order", [(2, 0), (3, 0), (3, 1), (4, 0), (6, 0), (7, 0), (20, 1), (31, 0), (32, 0), (33, 0), (239, 0), (240, 0), (359, 0), (360, 0)])
 def test_split_matches_three_kernels(layer, nb, order, zipf):
     lib = M.lib()
     M.check(lib.mmoe_set_bias(L, M.ptr(layer.bias) if zipf else None), "bias")
@@ -43,10 +44,10 @@ def test_split_matches_three_kernels(layer, nb, order, zipf):
             xg = x.copy()
             M.check(lib.mmoe_moe(L, M.ptr(hn), nb, M.ptr(xg), order), "mmoe_moe")
             plan = M.read_plan()
-            out[fused] = [xg] + [M.read(n, (nb * 8, k), t) for n, k, t in ITEMS] + [plan["ue"], plan["ustart"], np.array([plan["nu"], plan["np"], plan["tn"]])]
+            out[fused] = [xg] + [M.read(n, (nb * 8, k), t) for n, k, t in ITEMS] + [plan["ue"], plan["ustart"], np.array([plan["nu"], plan["np"]])]
         if zipf and nb >= 20:
             assert np.diff(out[1][-2]).max() > 16
-        for name, a, b in zip(["x"] + [i[0] for i in ITEMS] + ["ue", "ustart", "nu np tn"], out[0], out[1]):
+        for name, a, b in zip(["x"] + [i[0] for i in ITEMS] + ["ue", "ustart", "nu np"], out[0], out[1]):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"{name} differs"
     finally:
         M.check(lib.mmoe_set_debug(0), "debug off")
@@ -56,19 +57,19 @@ def test_split_matches_three_kernels(layer, nb, order, zipf):
 @pytest.fixture(scope="module")
 def slots(layer):
     lib = M.lib()
-    M.check(lib.gpux_init(1, 193), "gpux_init")
-    for s in range(193):
+    M.check(lib.gpux_init(1, 256), "gpux_init")
+    for s in range(256):
         lib.gpux_upload(0, s, *[M.ptr(a) for a in M.expert_views(layer.blk, s)])
 
 
-@pytest.mark.parametrize("sizes", [[1], [1] * 24, [17] + [1] * 23, [2] * 48, [17] + [2] * 47, [1] * 192, [17, 16] + [1] * 190])
+@pytest.mark.parametrize("sizes", [[1], [1] * 24, [17] + [1] * 23, [2] * 48, [17] + [2] * 47, [1] * 192, [17, 16] + [1] * 190, [17] + [1] * 255])
 def test_split_host_grouping(slots, sizes):
     """runs of the given lengths (17 pairs are two tiles) over 40 tokens through gpux_begin_multi"""
     lib = M.lib()
     nu, np_, nb = len(sizes), sum(sizes), 40
     _, hn = normed_hidden(SEED, 5300, nb)
     rng = np.random.default_rng(nu)
-    sl = rng.permutation(193)[:nu].astype(np.int32)
+    sl = rng.permutation(256)[:nu].astype(np.int32)
     ps = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
     pt = np.concatenate([np.sort(rng.permutation(nb)[:k]) for k in sizes]).astype(np.int32)
     out = {}
