@@ -472,105 +472,106 @@ __global__ void __launch_bounds__(256) k_router_chains2(const float *__restrict_
     }
 }
 
-// Large batches (batch order, NCH = 8) as a register-tiled GEMM that keeps maple.c's chains: one thread
-// owns one chain j for a TPT-token x 8-expert tile (independent FMA chains in registers), a block
-// covers 4 TPT tokens x 64 experts x 8 chains. Operands sit in LDS chain-major, hs[j][m][token] and
-// ws[j][m][expert] for column j + 8m, so a chain step reads 2 + 2 16-byte words. The router comes
-// pre-converted to fp32 in that order, wT[j][m][e] = w[e][j + 8m] (k_router_chain8_f32). Columns advance
-// in chunks of RG_MC steps, the next chunk loaded into registers while the current one is used.
-// After the last column the 8 chain values meet in LDS and are folded by hsum8.
-#define RG_BE 64
-#define RG_MC 16
-__global__ void k_router_chain8_f32(const uint16_t *__restrict__ w, float *__restrict__ wT) {
-    int i = blockIdx.x * 256 + threadIdx.x;          // over wT: [8][256][256]
-    int j = i >> 16, m = (i >> 8) & 255, e = i & 255;
-    wT[i] = bf16f(w[(size_t)e * MH + j + 8 * m]);
+// All logits exact for 240 tokens and more (batch order, 8 chains; from 1024 on where exact logits are asked for) on
+// v_mfma_f32_16x16x4_f32, which adds its 4 products one by one in ascending k, each as a fused multiply-add rounded to
+// nearest (attn.h): chain j of a logit is the product over columns j, j + 8, ... in order, so maple.c's sums come out bit
+// for bit. A workgroup of 8 waves takes 16 tokens x 32 experts, wave j its chain j for two fragments of 16 experts: 64
+// steps of 4 columns, two independent accumulators. The router (bf16, widened in registers) comes in the order the lanes
+// load it (k_router_frag), 8 steps a load; the tokens' rows in 8 chunks of 256 columns through two LDS stages, chain-major:
+// [token][chain j][g][s] for column 8 (4 s + g) + j, so a lane's operands of 4 steps are one 16-byte read. The 8 chain
+// values meet in LDS and are folded by hsum8.
+// Bound: load latency while one workgroup sits on a CU (to 512 tokens), then the f32 MFMA issue with one widening VALU
+// instruction each (T = 2048: 1.07 G FMAs, 14 us at the 75 T FMA/s of registers alone; the two do not overlap).
+// Measured (us, 333 / 700 / 2048 tokens): 10.6 / 14.4 / 27; a VALU tile of 16 tokens x 64 experts - / 32 / 42;
+// k_router_chains2 (with its top-8 and quantisation, 4.8 as a launch) 19.3 / - / -. 512-column chunks 10.6 / 14.8 / 29,
+// one expert fragment 12 / 15.7 / 36, 64 experts 15.6 / 16 / 26.8, 32 tokens x 64 experts 24 / 23.9 / 26.5.
+#define RF_ET 2
+#define RF_CC 256
+// wm[et][j][S][lane][t] = w[16 et + m][8 (4 (8 S + t) + g) + j], lane = (g, m)
+__global__ void k_router_frag(const uint16_t *__restrict__ w, uint16_t *__restrict__ wm) {
+    int i = blockIdx.x * 256 + threadIdx.x;      // over 256 * 2048 elements of wm
+    int t = i & 7, m = (i >> 3) & 15, g = (i >> 7) & 3, S = (i >> 9) & 7, j = (i >> 12) & 7, et = i >> 15;
+    wm[i] = w[(size_t)(16 * et + m) * MH + 8 * (4 * (8 * S + t) + g) + j];
 }
-// TPT tokens per thread: the block covers BT = 4 TPT tokens (TPT = 4: 16 tokens, 512 blocks at T = 2048 and
-// 32 accumulators per thread, so two or more waves share a SIMD).
-template <int TPT>
-__global__ void __launch_bounds__(256) k_router_gemm(const float *__restrict__ hn, int nb, const float *__restrict__ wT,
-                                                     const float *__restrict__ bias, float *__restrict__ rl) {
-    constexpr int BT = 4 * TPT, HP = BT + 4;        // tokens per block; token stride of hs (padded, 16-byte aligned)
-    constexpr int NH = BT * 128 / 4 / 256;           // float4 pieces of the token chunk per thread
-    constexpr int SM_CHUNK = 8 * RG_MC * HP + 8 * RG_MC * RG_BE, SM_RED = 8 * BT * RG_BE;
-    __shared__ __attribute__((aligned(16))) float smem[SM_CHUNK > SM_RED ? SM_CHUNK : SM_RED];
-    float *hs = smem, *ws = smem + 8 * RG_MC * HP;
-    int t = threadIdx.x, j = t >> 5, tg = (t >> 3) & 3, eg = t & 7;
-    int b0 = blockIdx.x * BT, e0 = blockIdx.y * RG_BE;
-    static_assert(RG_BE == 64, "the output loop gives thread t expert e0 + t % 64 in every round");
-    float be = 0.0f;
-    if (bias) be = bias[e0 + (t & 63)];   // loaded at entry, added to the thread's logits at the end
-    typedef float f4v __attribute__((ext_vector_type(4)));
-    f4v hr[NH], wr[8];
-    float acc[TPT][8];
+__global__ void __launch_bounds__(512, 4) k_router_f32(const float *__restrict__ hn, int nb, const uint16_t *__restrict__ wm,
+                                                       const float *__restrict__ bias, float *__restrict__ rl) {
+    constexpr int ET = RF_ET, CC = RF_CC;
+    // LDS floats per chain of a token's chunk (4 of padding) and per token: NS = 4 mod 64, so 16 rows' 16-byte reads meet in no bank
+    constexpr int JS = CC / 8 + 4, NS = 8 * JS + 36, NCK = MH / CC, ST = 16 * NS;
+    constexpr int QT = 512 / 16, NLD = CC / 4 / QT;   // staging: QT threads a row, NLD float4 each
+    __shared__ __attribute__((aligned(16))) float hs[2 * ST];
+    static_assert(CC == 256 && 8 * ET * 256 <= ST, "one 8-step router load a chunk; the chain values meet in one stage");
+    int tid = threadIdx.x, l = tid & 63, g = l >> 4, n = l & 15, j = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int t0 = blockIdx.x * 16, et0 = blockIdx.y * ET;
+    // staging: thread -> row tid / QT, columns 4 (tid % QT) + 4 QT i + u of the chunk
+    int sn = tid / QT, sq = tid % QT;
+    const float *src = hn + (size_t)min(t0 + sn, nb - 1) * MH + sq * 4;
+    const gptr_u4 *wp = (const gptr_u4 *)wm + (size_t)(et0 * 8 + j) * 8 * 64 + l;   // fragment e, group S at wp[(e * 64 + S) * 64]
+    v4f hr[NLD];
+    v4i wa[ET], wb[ET];
+    auto load_h = [&](int ch) {
 #pragma unroll
-    for (int a = 0; a < TPT; a++)
+        for (int i = 0; i < NLD; i++) hr[i] = *(const gptr_f4 *)(src + ch * CC + i * QT * 4);
+    };
+    auto store_h = [&](int b) {
 #pragma unroll
-        for (int b = 0; b < 8; b++) acc[a][b] = 0.0f;
-#define RG_LOAD(cn)                                                                                             \
-    {                                                                                                           \
-        _Pragma("unroll") for (int k = 0; k < NH; k++) {                                                        \
-            int idx = t + 256 * k, b = idx >> 5, c4 = idx & 31;                                                 \
-            hr[k] = *(const f4v *)(hn + (size_t)min(b0 + b, nb - 1) * MH + (cn) + 4 * c4);                      \
-        }                                                                                                       \
-        _Pragma("unroll") for (int k = 0; k < 8; k++) {                                                         \
-            int idx = t + 256 * k, jj = idx >> 8, mm = (idx >> 4) & 15, e4 = idx & 15;                          \
-            wr[k] = *(const f4v *)(wT + ((size_t)jj * 256 + (cn) / 8 + mm) * 256 + e0 + 4 * e4);                 \
-        }                                                                                                       \
-    }
-    RG_LOAD(0);
-    for (int c0 = 0; c0 < MH; c0 += 8 * RG_MC) {
-        __syncthreads();                             // the previous chunk is no longer read
+        for (int i = 0; i < NLD; i++) {
+            int c8 = (sq + i * QT) >> 1;   // column / 8 = 4 s + g
+            float *d = hs + b * ST + sn * NS + (sq & 1) * 4 * JS + (c8 & 3) * (CC / 32) + (c8 >> 2);
 #pragma unroll
-        for (int k = 0; k < NH; k++) {
-            int idx = t + 256 * k, b = idx >> 5, c4 = idx & 31;
-            int c = 4 * c4, base = (c >> 3) * HP + b, j0 = c & 7;
-            hs[((j0 + 0) * RG_MC) * HP + base] = hr[k].x;
-            hs[((j0 + 1) * RG_MC) * HP + base] = hr[k].y;
-            hs[((j0 + 2) * RG_MC) * HP + base] = hr[k].z;
-            hs[((j0 + 3) * RG_MC) * HP + base] = hr[k].w;
+            for (int u = 0; u < 4; u++) d[u * JS] = hr[i][u];
         }
+    };
+    auto load_w = [&](v4i (&w)[ET], int ch) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            int idx = t + 256 * k, jj = idx >> 8, mm = (idx >> 4) & 15, e4 = idx & 15;
-            *(f4v *)(ws + (jj * RG_MC + mm) * RG_BE + 4 * e4) = wr[k];
+        for (int e = 0; e < ET; e++) w[e] = wp[(e * 64 + ch) * 64];
+    };
+    v4f acc[ET];
+#pragma unroll
+    for (int e = 0; e < ET; e++) acc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto chunk = [&](int b, const v4i (&w)[ET]) {
+        const float *hp = hs + b * ST + n * NS + j * JS + g * (CC / 32);
+#pragma unroll
+        for (int s4 = 0; s4 < CC / 128; s4++) {   // 4 steps
+            v4f h4 = *(const v4f *)(hp + s4 * 4);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < ET; e++) {
+                    v4i v = w[e];
+                    int d = s4 * 2 + (q >> 1);
+                    uint32_t x = (uint32_t)(d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w);
+                    float wf = __uint_as_float((q & 1) ? x & 0xffff0000u : x << 16);
+                    acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf, h4[q], acc[e], 0, 0, 0);
+                }
         }
+    };
+    load_h(0);
+    load_w(wa, 0);
+    store_h(0);
+    load_h(1);
+    load_w(wb, 1);
+    __syncthreads();
+#pragma unroll
+    for (int ch = 0; ch < NCK; ch++) {
+        chunk(ch & 1, ch & 1 ? wb : wa);
+        if (ch == NCK - 1) break;
+        store_h((ch + 1) & 1);   // the stage of chunk ch - 1, read by nobody since the last barrier
+        if (ch < NCK - 2) { load_h(ch + 2); load_w(ch & 1 ? wb : wa, ch + 2); }
         __syncthreads();
-        if (c0 + 8 * RG_MC < MH) RG_LOAD(c0 + 8 * RG_MC);
-#pragma unroll 4
-        for (int m = 0; m < RG_MC; m++) {
-            const float *hp = hs + (j * RG_MC + m) * HP + tg * TPT, *wp = ws + (j * RG_MC + m) * RG_BE + eg * 8;
-            float hv[TPT];
-#pragma unroll
-            for (int a = 0; a < TPT; a += 4) { float4 h = *(const float4 *)(hp + a); hv[a] = h.x; hv[a + 1] = h.y; hv[a + 2] = h.z; hv[a + 3] = h.w; }
-            float4 w0 = *(const float4 *)wp, w1 = *(const float4 *)(wp + 4);
-            float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-            for (int a = 0; a < TPT; a++)
-#pragma unroll
-                for (int b = 0; b < 8; b++) acc[a][b] = __builtin_fmaf(wv[b], hv[a], acc[a][b]);
-        }
     }
-#undef RG_LOAD
+    float *red = hs;   // [j][fragment][token][expert], in stage 0: NCK is even, it was last read before the last barrier
+#pragma unroll
+    for (int e = 0; e < ET; e++) *(v4f *)(red + ((j * ET + e) * 16 + n) * 16 + 4 * g) = acc[e];
     __syncthreads();
-    float *red = smem;                               // red[j][token][expert]
+    static_assert(ET == 2 && NCK % 2 == 0, "one logit a thread");
+    int m = tid & 15, e = (tid >> 4) & 1, tok = tid >> 5, ex = (et0 + e) * 16 + m;
+    float v[8];
 #pragma unroll
-    for (int a = 0; a < TPT; a++)
-#pragma unroll
-        for (int b = 0; b < 8; b += 4)
-            *(float4 *)(red + (j * BT + tg * TPT + a) * RG_BE + eg * 8 + b) = make_float4(acc[a][b], acc[a][b + 1], acc[a][b + 2], acc[a][b + 3]);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < BT * RG_BE / 256; q++) {
-        int o = q * 256 + t, tok = o >> 6, e = o & 63;
-        float v[8];
-#pragma unroll
-        for (int jj = 0; jj < 8; jj++) v[jj] = red[(jj * BT + tok) * RG_BE + e];
-        float r = hsum8(v);
-        if (bias) r = r + be;
-        if (b0 + tok < nb) rl[(size_t)(b0 + tok) * MNE + e0 + e] = r;
-    }
+    for (int jj = 0; jj < 8; jj++) v[jj] = red[((jj * ET + e) * 16 + tok) * 16 + m];
+    float r = hsum8(v);
+    if (bias) r = r + bias[ex];
+    if (t0 + tok < nb) rl[(size_t)(t0 + tok) * MNE + ex] = r;
 }
 
 // Large batches, approximate logits on the bf16 MFMA + exact refinement (k_refine_topk).
@@ -617,10 +618,9 @@ __global__ void __launch_bounds__(WAVES * 64) k_router_mfma(const uint16_t *__re
     constexpr int NT = WAVES * 64, ER = 32 * WAVES * EW;
     constexpr int NW = ER * 8 / NT;              // router pieces (16 bytes) staged per thread: rows wrow + (NT / 8) i
     constexpr int NH = 32 * 16 / NT;             // input pieces (4 floats) per thread: rows hrow + (NT / 16) i
-    // LDS stages (2 for the 8-wave block, one per CU anyway; 1 for the 4-wave block, several per CU): chunk ck
-    // is stored to stage ck % NB, so with 2 stages one barrier per chunk suffices (a stage is rewritten two chunks
-    // later, after every wave has passed the barrier of the chunk in between)
-    constexpr int NB = WAVES == 8 ? 2 : 1;
+    // two LDS stages (the 8-wave block is one per CU anyway): chunk ck is stored to stage ck % 2, so one barrier per chunk
+    // suffices (a stage is rewritten two chunks later, after every wave has passed the barrier of the chunk in between)
+    constexpr int NB = 2;
     __shared__ __attribute__((aligned(16))) uint16_t ws_[NB][ER * RM_LR];
     __shared__ __attribute__((aligned(16))) uint16_t hsl_[NB][RM_PARTS][32 * RM_LR];
     int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, r = l & 31, kg = l >> 5;
@@ -645,7 +645,6 @@ __global__ void __launch_bounds__(WAVES * 64) k_router_mfma(const uint16_t *__re
         const int q = ck % RM_PF;
         uint16_t *ws = ws_[ck % NB];
         uint16_t (*hsl)[32 * RM_LR] = hsl_[ck % NB];
-        if (NB == 1) __syncthreads();
 #pragma unroll
         for (int i = 0; i < NW; i++) *(v4i *)(&ws[(wrow + (NT / 8) * i) * RM_LR + wpc * 8]) = rw[q][i];
 #pragma unroll

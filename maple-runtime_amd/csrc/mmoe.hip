@@ -103,7 +103,7 @@ __global__ void k_fill_zero(int *p, int n) { int i = blockIdx.x * 256 + threadId
 // Global state
 // ------------------------------------------------------------------------------------------------------
 struct Region { const void *host; size_t len; uint8_t *dev; };
-struct LayerW { ExpPtr *tab = nullptr; uint16_t *router = nullptr; uint16_t *rc16 = nullptr, *rc8 = nullptr; float *rf8 = nullptr, *w1max = nullptr; uint16_t *post_ln = nullptr; float *bias = nullptr; };
+struct LayerW { ExpPtr *tab = nullptr; uint16_t *router = nullptr; uint16_t *rc16 = nullptr, *rc8 = nullptr; uint16_t *rm = nullptr; float *w1max = nullptr; uint16_t *post_ln = nullptr; float *bias = nullptr; };
 
 // Pinned host memory that kernels read and write in place (coherent): tables from the host in a ring of blocks, each reused
 // only after the launch that reads it has run, and one block for results. Sized for the largest grouping (2048 tokens).
@@ -162,7 +162,7 @@ static void kl(void (*f)(P...), dim3 g, dim3 b, size_t shm, A &&...a) {
 }
 
 // small (carved sets): at most 64 tokens, so only the decode and 16-token-tile paths run: no int16 down side
-// buffer (2048+ pairs only), no approximate-router buffers (512+ tokens), no host-side hidden state copy.
+// buffer (2048+ pairs only), no approximate-router buffers (1024+ tokens), no host-side hidden state copy.
 static int work_alloc(Work &w, int maxtok, Carve *c = nullptr) {
     if (maxtok < 1 || maxtok > MMOE_MAXTOK || (c && maxtok > 64)) { seterr("maxtok %d outside 1..%d", maxtok, c ? 64 : MMOE_MAXTOK); return -1; }
     w.maxtok = maxtok; w.maxp = maxtok * MTOPK;
@@ -256,16 +256,16 @@ static bool S_expert16 = true;   // tiles of 16: the fused kernels (else three k
 static int tile_tn(int np) { return np >= (S_expert16 ? 2880 : 2048) ? 64 : 16; }
 
 // Router logits of nb tokens (d_hn) with layer L's router; order 0 = batch (maple.c:853-889), 1 = step (bf_row)
-static bool S_router_exact = false;
+static bool S_router_exact = false;   // batches of 1024+: k_router_f32 (else MFMA logits + exact refinement)
 #ifndef ROUTER_TK
 #define ROUTER_TK 1
 #endif
 #ifndef ROUTER_TPB
 #define ROUTER_TPB 2   // tokens per block of the chain router with the top-8 tail (below 512 tokens)
 #endif
-static bool S_router_tk = ROUTER_TK;   // batches below 512: top-8 and quantisation in the router launch   // batches of 512+: MFMA logits + exact refinement (else the exact chain GEMM)
+static bool S_router_tk = ROUTER_TK;   // chain router: top-8 and quantisation in the router launch
 // exact_only: never the approximate large-batch router (callers that hand the logits themselves to the host)
-// tk (batches below 512 tokens): the router launch also runs each token's softmax/top-8 (per-chunk counts into
+// tk (the chain router): the router launch also runs each token's softmax/top-8 (per-chunk counts into
 // hist unless hist is null) and its int8 quantisation, in the last of the token's router blocks
 static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int order, bool exact_only, bool tk, int *hist) {
     LayerW &lw = S.layers[L];
@@ -274,6 +274,12 @@ static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int or
     if (!lw.router) { seterr("layer %d has no router (mmoe_set_layer)", L); return -1; }
     // w.norm_x set (stacked path): the chain routers form hn = rmsnorm(x, post_ln) into d_hn themselves
     float *hn_w = const_cast<float *>(d_hn);
+    // Every logit on the f32 MFMA, top-8 and quantisation in a launch of their own, for 240 tokens (where the grouping is a
+    // launch of its own as well) to 1023. Whole layers against the chain router with both in its tail, us: 200 tokens 66.9 /
+    // 67.5, 333: 82.8 / 86.0, 511: 97.4 / 104.4; against approximate logits on the bf16 MFMA with refinement: 512 97.5 / 101.5,
+    // 700 107.1 / 109.0, 1021 118.9 / 121.0, 1200 129.9 / 128.8. Larger batches where exact logits are asked for.
+    if (order == MMOE_ORDER_BATCH && !w.norm_x && nb >= 240 && (nb < 1024 || S_router_exact || exact_only))
+        return launch(MMOE_K_ROUTER, [&] { kl(k_router_f32, dim3((nb + 15) / 16, MNE / (16 * RF_ET)), 512, 0, d_hn, nb, lw.rm, lw.bias, w.rl); });
     if (tk && nb < 512) {
         RouteTail rt{w.top, w.tw, w.qx, w.qsx, w.qsumx, hist, w.rcnt};
         w.routed = true;
@@ -298,16 +304,13 @@ static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int or
         if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16, true>, dim3(MNE * 16 / 256, nb), 256, 0, w.norm_x, nb, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w, RouteTail{}); });
         return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16>, dim3(MNE * 16 / 256, nb), 256, 0, d_hn, nb, lw.rc16, lw.bias, w.rl, nullptr, nullptr, RouteTail{}); });
     }
-    if (nb < 512) {   // one block per (token, 32 experts): 8 nb blocks, router reread from L2 per token
+    if (nb < 240 || w.norm_x) {   // one block per (token, 32 experts): 8 nb blocks, router reread from L2 per token
         if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8, true>, dim3(MNE * 8 / 256, nb), 256, 0, w.norm_x, nb, lw.rc8, lw.bias, w.rl, w.norm_w, hn_w, RouteTail{}); });
         return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8>, dim3(MNE * 8 / 256, nb), 256, 0, d_hn, nb, lw.rc8, lw.bias, w.rl, nullptr, nullptr, RouteTail{}); });
     }
-    if (S_router_exact || exact_only)
-        return launch(MMOE_K_ROUTER, [&] { kl(k_router_gemm<4>, dim3((nb + 15) / 16, MNE / RG_BE), 256, 0, d_hn, nb, lw.rf8, lw.bias, w.rl); });
     // approximate logits on the bf16 MFMA; k_refine_topk makes the top-8 exact
     w.refine = true;
-    if (nb >= 1024) return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<8, 1>, dim3((nb + 31) / 32, MNE / 256, 4), 512, 0, lw.router, d_hn, nb, w.rpart); });
-    return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<4, 1>, dim3((nb + 31) / 32, MNE / 128, 4), 256, 0, lw.router, d_hn, nb, w.rpart); });
+    return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<8, 1>, dim3((nb + 31) / 32, MNE / 256, 4), 512, 0, lw.router, d_hn, nb, w.rpart); });
 }
 
 // the router launch, recording whether rl now holds every logit exactly (mmoe_route may then take them as they are)
@@ -315,7 +318,8 @@ static int stage_router(Work &w, int L, const float *d_hn, int nb, int order, bo
                         int *hist = nullptr) {
     w.rl_nb = 0;
     int rc = stage_router_launch(w, L, d_hn, nb, order, exact_only, tk, hist);
-    if (!rc && !w.refine) w.rl_nb = nb;
+    // (from 512 tokens mmoe_route takes them only from calls that ask for exact logits)
+    if (!rc && !w.refine && (order == MMOE_ORDER_STEP || nb < 512 || S_router_exact || exact_only)) w.rl_nb = nb;
     return rc;
 }
 
@@ -472,7 +476,7 @@ static int moe_dev(Work &w, int L, const float *d_hn, int nb, float *d_x, int or
     if (L < 0 || L >= NLMAX || !S.layers[L].tab) { seterr("layer %d not set (mmoe_set_layer)", L); return -1; }
     if (nb == 1 && S_dec_enabled) return moe_dec(w, L, d_hn, 0, d_x, order);
     int np = nb * MTOPK, tn = tile_tn(np);
-    // below 512 tokens the router launch also runs the top-8 and the quantisation; the per-chunk counts are for
+    // the chain router's launch also runs the top-8 and the quantisation; the per-chunk counts are for
     // k_group, which the fused small-tile kernel does without (it groups itself)
     bool grp16 = tn == 16 && S_expert16 && nb <= E16_GRP_MAXTOK;
     if (stage_router(w, L, d_hn, nb, order, false, S_router_tk, grp16 ? nullptr : w.hist)) return -1;
@@ -1010,8 +1014,8 @@ int mmoe_set_layer(int L, const uint32_t *loc, const int *regs, const uint16_t *
     return 0;
 }
 
-// Layer L's router (bf16 [256][2048]) into HBM with its chain-major copies (both orders, and fp32 for the
-// tiled batch router) and the bound the MFMA router option uses.
+// Layer L's router (bf16 [256][2048]) into HBM with its chain-major copies (both orders, and MFMA order
+// for k_router_f32) and the bound the MFMA router option uses.
 static int set_router(int L, const uint16_t *router) {
     if (mmoe_graph_reset()) return -1;
     LayerW &lw = S.layers[L];
@@ -1021,8 +1025,8 @@ static int set_router(int L, const uint16_t *router) {
     if (!lw.rc8) HC(hipMalloc(&lw.rc8, (size_t)MNE * MH * 2));
     kl(k_router_chainmajor<16>, MNE * MH / 256, 256, 0, lw.router, lw.rc16);
     kl(k_router_chainmajor<8>, MNE * MH / 256, 256, 0, lw.router, lw.rc8);
-    if (!lw.rf8) HC(hipMalloc(&lw.rf8, (size_t)MNE * MH * 4));
-    kl(k_router_chain8_f32, MNE * MH / 256, 256, 0, lw.router, lw.rf8);
+    if (!lw.rm) HC(hipMalloc(&lw.rm, (size_t)MNE * MH * 2));
+    kl(k_router_frag, MNE * MH / 256, 256, 0, lw.router, lw.rm);
     if (!lw.w1max) HC(hipMalloc(&lw.w1max, 2 * sizeof(float)));
     kl(k_router_l1max, 1, 256, 0, lw.router, lw.w1max);
     HC(hipGetLastError());
@@ -1116,7 +1120,8 @@ int mmoe_stack_dev(int L0, int nl, float *d_x, int nb, int order) {
         if (L < 0 || L >= NLMAX || !S.layers[L].tab) { seterr("mmoe_stack_dev: layer %d not set", L); return -1; }
         if (nb == 1 && S_dec_enabled) { if (moe_dec(w, L, d_x, 1, d_x, order)) return -1; continue; }
         const uint16_t *pw = S.layers[L].post_ln;
-        if (order == MMOE_ORDER_STEP || nb < 512) {   // the chain router forms hn itself (no rmsnorm launch)
+        // the chain router forms hn itself, which saves the rmsnorm launch (4.5 us); from 384 tokens k_router_f32 gains more
+        if (order == MMOE_ORDER_STEP || nb < 384) {
             w.norm_x = d_x; w.norm_w = pw;
             int rc = moe_dev(w, L, w.hn, nb, d_x, order);
             w.norm_x = nullptr; w.norm_w = nullptr;
