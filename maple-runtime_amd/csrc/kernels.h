@@ -1021,12 +1021,21 @@ struct HostGroup { const ExpPtr *ep; const int *ustart, *ptok; const float *pw; 
 __global__ void __launch_bounds__(256) k_host_group(HostGroup h, int ncopy, Plan *__restrict__ plan, int tn, Tile *__restrict__ tiles,
                                                     DnTile *__restrict__ dt, ExpPtr *__restrict__ eptr, int *__restrict__ utok,
                                                     float *__restrict__ uw, int *__restrict__ tp, const float *__restrict__ x, int nb,
-                                                    int8_t *__restrict__ qx, float *__restrict__ qsx, int *__restrict__ qsumx) {
+                                                    float *__restrict__ hn, int8_t *__restrict__ qx, float *__restrict__ qsx, int *__restrict__ qsumx) {
     __shared__ int wt[4];
     int t = threadIdx.x, l = t & 63, wv = t >> 6;
     if ((int)blockIdx.x > ncopy) {
         int row = ((int)blockIdx.x - 1 - ncopy) * 4 + wv;
-        if (row < nb) quant_wave<MH>(x + (size_t)row * MH, l, qx + (size_t)row * MH, qsx + row, qsumx + row);
+        if (row < nb) {
+            if (hn) {   // rows from the host: the work input in device memory as well
+                v4f v[MH / 256];
+#pragma unroll
+                for (int i = 0; i < MH / 256; i++) v[i] = ((const v4f *)(x + (size_t)row * MH))[l + 64 * i];
+#pragma unroll
+                for (int i = 0; i < MH / 256; i++) ((v4f *)(hn + (size_t)row * MH))[l + 64 * i] = v[i];
+            }
+            quant_wave<MH>(x + (size_t)row * MH, l, qx + (size_t)row * MH, qsx + row, qsumx + row);
+        }
         return;
     }
     if (blockIdx.x) {   // words: the pointers, then ptok, pw, tp
@@ -1061,6 +1070,12 @@ __global__ void __launch_bounds__(256) k_host_group(HostGroup h, int ncopy, Plan
             plan->nu = nu; plan->np = p0 + c; plan->ntile_gu = ist; plan->tn = tn;
         }
     }
+}
+
+// up to 64 used experts' pointers from the kernel's own arguments (captured calls)
+struct ExpPtr64 { ExpPtr e[64]; };
+__global__ void __launch_bounds__(64) k_put_eptr(ExpPtr64 p, int n, ExpPtr *__restrict__ eptr) {
+    if ((int)threadIdx.x < n) eptr[threadIdx.x] = p.e[threadIdx.x];
 }
 
 // The routing results of nb tokens (mmoe_route) into one run of pinned host memory, [nu, ue 256, ustart 257] then top, tw,

@@ -507,27 +507,47 @@ static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, 
     if (tp) for (int i = 0; i < nb * MTOPK; i++) if (tp[i] < 0 || tp[i] >= np) { seterr("tp[%d] = %d outside 0..%d", i, tp[i], np - 1); return -1; }
     int tn = tile_tn(np), ntile = 0;
     for (int u = 0; u < nu; u++) ntile += (ustart[u + 1] - ustart[u] + tn - 1) / tn;
-    HostRing &r = S.hs[S.hs_next];
-    S.hs_next = (S.hs_next + 1) % HS_RING;
-    if (r.used) HC(hipEventSynchronize(r.ev));
-    uint8_t *q = r.p;
-    auto put = [&](const void *src, size_t n) { void *d = q; memcpy(d, src, n); q += (n + 15) / 16 * 16; return d; };
     HostGroup h{};
-    h.ep = (const ExpPtr *)put(eptr_h, sizeof(ExpPtr) * nu);
-    h.ustart = (const int *)put(ustart, sizeof(int) * (nu + 1));
-    h.ptok = (const int *)put(ptok, sizeof(int) * np);
-    if (pw) h.pw = (const float *)put(pw, sizeof(float) * np);
-    if (tp) h.tp = (const int *)put(tp, sizeof(int) * nb * MTOPK);
+    h.nu = nu; h.np = np; h.ntp = tp ? nb * MTOPK : 0;
     const float *x = w.hn;
     size_t xb = (size_t)nb * MH * 4;
-    if (x_h && xb <= HS_X) x = (const float *)put(x_h, xb);
-    else if (x_h) HC(hipMemcpyAsync(w.hn, x_h, xb, hipMemcpyHostToDevice, S.st));
-    h.nu = nu; h.np = np; h.ntp = tp ? nb * MTOPK : 0;
-    int words = nu * (int)(sizeof(ExpPtr) / 4) + np + (pw ? np : 0) + h.ntp, ncopy = std::min((words + 1023) / 1024, 64);
+    int ncopy = 0;
+    HostRing *r = nullptr;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HC(hipStreamIsCapturing(S.st, &cs));
+    if (cs != hipStreamCaptureStatusNone) {
+        // A captured call reads its tables when the graph runs: from the caller's arrays, not from a block of the ring that
+        // later calls fill again. The pointers, made here on the stack, travel as kernel arguments.
+        for (int u = 0; u < nu; u += 64) {
+            ExpPtr64 e;
+            memcpy(e.e, eptr_h + u, sizeof(ExpPtr) * std::min(nu - u, 64));
+            if (launch(MMOE_K_GROUP, [&] { kl(k_put_eptr, 1, 64, 0, e, std::min(nu - u, 64), w.eptr + u); })) return -1;
+        }
+        HC(hipMemcpyAsync(w.ustart, ustart, sizeof(int) * (nu + 1), hipMemcpyHostToDevice, S.st));
+        HC(hipMemcpyAsync(w.utok, ptok, sizeof(int) * np, hipMemcpyHostToDevice, S.st));
+        if (pw) HC(hipMemcpyAsync(w.uw, pw, sizeof(float) * np, hipMemcpyHostToDevice, S.st));
+        if (tp) HC(hipMemcpyAsync(w.tp, tp, sizeof(int) * nb * MTOPK, hipMemcpyHostToDevice, S.st));
+        if (x_h) HC(hipMemcpyAsync(w.hn, x_h, xb, hipMemcpyHostToDevice, S.st));
+        h.ep = w.eptr; h.ustart = w.ustart; h.ptok = w.utok;
+    } else {
+        r = &S.hs[S.hs_next];
+        S.hs_next = (S.hs_next + 1) % HS_RING;
+        if (r->used) HC(hipEventSynchronize(r->ev));
+        uint8_t *q = r->p;
+        auto put = [&](const void *src, size_t n) { void *d = q; memcpy(d, src, n); q += (n + 15) / 16 * 16; return d; };
+        h.ep = (const ExpPtr *)put(eptr_h, sizeof(ExpPtr) * nu);
+        h.ustart = (const int *)put(ustart, sizeof(int) * (nu + 1));
+        h.ptok = (const int *)put(ptok, sizeof(int) * np);
+        if (pw) h.pw = (const float *)put(pw, sizeof(float) * np);
+        if (tp) h.tp = (const int *)put(tp, sizeof(int) * nb * MTOPK);
+        if (x_h && xb <= HS_X) x = (const float *)put(x_h, xb);
+        else if (x_h) HC(hipMemcpyAsync(w.hn, x_h, xb, hipMemcpyHostToDevice, S.st));
+        int words = nu * (int)(sizeof(ExpPtr) / 4) + np + (pw ? np : 0) + h.ntp;
+        ncopy = std::min((words + 1023) / 1024, 64);
+    }
     if (launch(MMOE_K_GROUP, [&] { kl(k_host_group, 1 + ncopy + (nb + 3) / 4, 256, 0, h, ncopy, w.plan, tn, w.tiles, tn == 16 ? w.dt : (DnTile *)nullptr,
-                                      w.eptr, w.utok, w.uw, w.tp, x, nb, w.qx, w.qsx, w.qsumx); })) return -1;
-    HC(hipEventRecord(r.ev, S.st));
-    r.used = true;
+                                      w.eptr, w.utok, w.uw, w.tp, x, nb, x == w.hn ? nullptr : w.hn, w.qx, w.qsx, w.qsumx); })) return -1;
+    if (r) { HC(hipEventRecord(r->ev, S.st)); r->used = true; }
     return stage_experts(w, np, nu, tn, false, ntile);
 }
 

@@ -95,3 +95,61 @@ def test_kv_copied_beside_the_stack(model):
     lib.gfull_begin(M.ptr(xs[0]), 200, 0)
     M.check(lib.mmoe_gfull_stack(0, NL), "stack"); M.check(lib.mmoe_gfull_stack(0, NL), "stack")
     assert np.array_equal(twice, read_kv(lib, 200)) and not np.array_equal(twice, want[0])
+
+
+@pytest.mark.parametrize("nb", [3, 8, 9])
+def test_work_input_after_gpre_moe(model, nb):
+    """the call's rows are in the work input (mmoe_read) whichever way they reached the card"""
+    lib, rids = model
+    rng = np.random.default_rng(SEED + 83 + nb)
+    g = O.group(np.argsort(rng.random((nb, 256)), 1)[:, :8].astype(np.int32), rng.random((nb, 8)).astype(np.float32))
+    x = rng.standard_normal((nb, H)).astype(np.float32)
+    y, regs = np.empty_like(x), np.array([rids[0], -1, -1, -1], np.int32)
+    loc, tp = M.block_loc(0, list(g["ue"])), np.ascontiguousarray(g["tp"])
+    assert lib.gpre_moe(M.ptr(x), nb, g["nu"], M.ptr(loc), M.ptr(regs), None, M.ptr(g["ustart"]), M.ptr(g["utok"]), M.ptr(g["uw"]),
+                        M.ptr(tp), M.ptr(y)) >= 0
+    assert np.array_equal(M.read("HN", (nb, H), np.float32).view(np.int32), x.view(np.int32))
+
+
+@pytest.mark.parametrize("nb", [6, 40])
+def test_grouping_under_capture(model, nb):
+    """a captured gfull_moe call, replayed with eager calls of other groupings (more than the ring holds) in between"""
+    lib, rids = model
+    hip = C.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(SEED + 90 + nb)
+    calls = []
+    for k in range(6):
+        g = O.group(np.argsort(rng.random((nb, 256)), 1)[:, :8].astype(np.int32), rng.random((nb, 8)).astype(np.float32))
+        calls.append((g, M.block_loc(0, list(g["ue"])), np.array([rids[k % NL], -1, -1, -1], np.int32), np.ascontiguousarray(g["tp"])))
+    x0 = rng.standard_normal((nb, H)).astype(np.float32)
+
+    def call(k):
+        g, loc, regs, tp = calls[k]
+        lib.gfull_moe(g["nu"], M.ptr(loc), M.ptr(regs), M.ptr(g["ustart"]), M.ptr(g["utok"]), M.ptr(g["uw"]), M.ptr(tp))
+
+    def read():
+        x = np.empty((nb, H), np.float32)
+        lib.gfull_read(M.ptr(x), None)
+        return x
+
+    lib.gfull_begin(M.ptr(x0), nb, 0)
+    assert lib.mmoe_gfull_post_norm(0, None) == 0
+    for k in (*range(6), 0):
+        call(k)
+    want = read()
+    stream, graph, ex = C.c_void_p(lib.mmoe_stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    call(0)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    try:
+        for _ in range(3):
+            lib.gfull_begin(M.ptr(x0), nb, 0)
+            assert lib.mmoe_gfull_post_norm(0, None) == 0
+            for k in range(6):
+                call(k)
+            assert hip.hipGraphLaunch(ex, stream) == 0
+            assert np.array_equal(read().view(np.int32), want.view(np.int32))
+    finally:
+        M.check(lib.mmoe_sync(), "sync")
+        hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
