@@ -287,11 +287,11 @@ def full_prefill(lib, rids, args):
             log(f"  {k:12s} {tt / n * 1e3:8.2f} us avg x {n}")
         # scores and weighted sum: 16 heads x 128 dims x (window length) fp32 FMAs per token each, in maple.c's
         # order on the f32 matrix cores; averaged over the 24 layers (every fourth global, the rest a 512-position
-        # window), against the fp32 FMA peak of the vector units without packed operations
+        # window), against the fp32 FMA peak of the matrix units
         pos = np.arange(pos0, pos0 + T)
         win_len = {0: np.minimum(pos, 512) + 1, 1: pos + 1}
         fma = sum(16 * 128 * int(win_len[int(L % 4 == 3)].sum()) for L in range(NL)) / NL
-        fma_peak = 256 * 4 * 16 * 2.4e9
+        fma_peak = 256 * 4 * 32 * 2.4e9   # fp32 matrix units: 32 FMAs per SIMD and cycle, twice the VALU
         att_core = sum(fk[k][0] for k in ("att_scores", "att_softmax", "att_pv") if k in fk) / NL   # ms per layer
         frac = round(2 * fma / (att_core * 1e-3) / fma_peak, 4)
         key = "first_chunk" if pos0 == 0 else "second_chunk"
