@@ -133,7 +133,7 @@ int mmoe_moe_dev_noalloc(int L, const float *d_hn, int nb, float *d_x, int order
 /* Routing only, in place of maple.c's job_topk + group_pairs (maple.c:910-938) and the tp table its callers
  * build (maple.c:762, 1019), for a caller that keeps its own gpre_moe / gfull_moe (maple.c:763, 1021): rl[nb][256]
  * router logits (host), or NULL for the logits the last router call left on the device (gfull_attn,
- * mmoe_gfull_post_norm, and mmoe_moe* below 512 tokens or with
+ * mmoe_gfull_post_norm, and mmoe_moe* when every logit was computed exactly: below 512 tokens or with
  * mmoe_set_router_mode(1)); NULL is refused with -1 unless that call covered exactly nb tokens.
  * -> maple.c's TOPB/TWB (top[nb][8], tw[nb][8]: softmax, the 8 largest p in pick order, renormalised), the pairs grouped by expert (ue[nu] used experts ascending, ustart[nu+1], utok[nb*8] and
  * uw[nb*8] = UTOK/UW) and tp[nb][8] (each token's pair ids, ascending). Any output may be NULL. Synchronous;
@@ -192,8 +192,8 @@ int mmoe_set_decode_path(int on);
  * (few experts: gate/up and down with the act quantisation, each expert over many workgroups; else one kernel per
  * tile), 0 = the three separate kernels. All give identical results. */
 int mmoe_set_expert_path(int fused);
-/* Router of batches of >= 1024 tokens in batch order (smaller ones: every logit exact): 0 (default) = bf16 MFMA logits on the input split into
- * three exact bf16 parts, with every expert that a rounding bound cannot exclude from a token's top 8 recomputed
+/* Router of batches of >= 512 tokens in batch order (smaller ones: every logit exact): 0 (default) = bf16 MFMA logits on the
+ * two leading bf16 parts of each input value, with every expert that a rounding bound cannot exclude from a token's top 8 recomputed
  * in maple.c's exact chain order (top-8 indices and their logits stay maple.c's; the other logits, and through
  * the softmax sum the weights, differ by about 1e-7); 1 = exact fp32 FMA chains for every logit. gfull_attn's
  * logits, which maple.c consumes itself, always use the exact chains. */

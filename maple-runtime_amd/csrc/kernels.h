@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(256) k_router_chains2(const float *__restrict_
     }
 }
 
-// All logits exact for 240 tokens and more (batch order, 8 chains; from 1024 on where exact logits are asked for) on
+// All logits exact for 240 tokens and more (batch order, 8 chains; from 512 on where exact logits are asked for) on
 // v_mfma_f32_16x16x4_f32, which adds its 4 products one by one in ascending k, each as a fused multiply-add rounded to
 // nearest (attn.h): chain j of a logit is the product over columns j, j + 8, ... in order, so maple.c's sums come out bit
 // for bit. A workgroup of 8 waves takes 16 tokens x 32 experts, wave j its chain j for two fragments of 16 experts: 64
@@ -618,9 +618,10 @@ __global__ void __launch_bounds__(WAVES * 64) k_router_mfma(const uint16_t *__re
     constexpr int NT = WAVES * 64, ER = 32 * WAVES * EW;
     constexpr int NW = ER * 8 / NT;              // router pieces (16 bytes) staged per thread: rows wrow + (NT / 8) i
     constexpr int NH = 32 * 16 / NT;             // input pieces (4 floats) per thread: rows hrow + (NT / 16) i
-    // two LDS stages (the 8-wave block is one per CU anyway): chunk ck is stored to stage ck % 2, so one barrier per chunk
-    // suffices (a stage is rewritten two chunks later, after every wave has passed the barrier of the chunk in between)
-    constexpr int NB = 2;
+    // LDS stages (2 for the 8-wave block, one per CU anyway; 1 for the 4-wave block, several per CU): chunk ck
+    // is stored to stage ck % NB, so with 2 stages one barrier per chunk suffices (a stage is rewritten two chunks
+    // later, after every wave has passed the barrier of the chunk in between)
+    constexpr int NB = WAVES == 8 ? 2 : 1;
     __shared__ __attribute__((aligned(16))) uint16_t ws_[NB][ER * RM_LR];
     __shared__ __attribute__((aligned(16))) uint16_t hsl_[NB][RM_PARTS][32 * RM_LR];
     int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, r = l & 31, kg = l >> 5;
@@ -645,6 +646,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_router_mfma(const uint16_t *__re
         const int q = ck % RM_PF;
         uint16_t *ws = ws_[ck % NB];
         uint16_t (*hsl)[32 * RM_LR] = hsl_[ck % NB];
+        if (NB == 1) __syncthreads();
 #pragma unroll
         for (int i = 0; i < NW; i++) *(v4i *)(&ws[(wrow + (NT / 8) * i) * RM_LR + wpc * 8]) = rw[q][i];
 #pragma unroll

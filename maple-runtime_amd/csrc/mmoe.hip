@@ -162,7 +162,7 @@ static void kl(void (*f)(P...), dim3 g, dim3 b, size_t shm, A &&...a) {
 }
 
 // small (carved sets): at most 64 tokens, so only the decode and 16-token-tile paths run: no int16 down side
-// buffer (2048+ pairs only), no approximate-router buffers (1024+ tokens), no host-side hidden state copy.
+// buffer (2048+ pairs only), no approximate-router buffers (512+ tokens), no host-side hidden state copy.
 static int work_alloc(Work &w, int maxtok, Carve *c = nullptr) {
     if (maxtok < 1 || maxtok > MMOE_MAXTOK || (c && maxtok > 64)) { seterr("maxtok %d outside 1..%d", maxtok, c ? 64 : MMOE_MAXTOK); return -1; }
     w.maxtok = maxtok; w.maxp = maxtok * MTOPK;
@@ -256,7 +256,7 @@ static bool S_expert16 = true;   // tiles of 16: the fused kernels (else three k
 static int tile_tn(int np) { return np >= (S_expert16 ? 2880 : 2048) ? 64 : 16; }
 
 // Router logits of nb tokens (d_hn) with layer L's router; order 0 = batch (maple.c:853-889), 1 = step (bf_row)
-static bool S_router_exact = false;   // batches of 1024+: k_router_f32 (else MFMA logits + exact refinement)
+static bool S_router_exact = false;   // batches of 512+: k_router_f32 (else MFMA logits + exact refinement)
 #ifndef ROUTER_TK
 #define ROUTER_TK 1
 #endif
@@ -274,11 +274,13 @@ static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int or
     if (!lw.router) { seterr("layer %d has no router (mmoe_set_layer)", L); return -1; }
     // w.norm_x set (stacked path): the chain routers form hn = rmsnorm(x, post_ln) into d_hn themselves
     float *hn_w = const_cast<float *>(d_hn);
-    // Every logit on the f32 MFMA, top-8 and quantisation in a launch of their own, for 240 tokens (where the grouping is a
-    // launch of its own as well) to 1023. Whole layers against the chain router with both in its tail, us: 200 tokens 66.9 /
-    // 67.5, 333: 82.8 / 86.0, 511: 97.4 / 104.4; against approximate logits on the bf16 MFMA with refinement: 512 97.5 / 101.5,
-    // 700 107.1 / 109.0, 1021 118.9 / 121.0, 1200 129.9 / 128.8. Larger batches where exact logits are asked for.
-    if (order == MMOE_ORDER_BATCH && !w.norm_x && nb >= 240 && (nb < 1024 || S_router_exact || exact_only))
+    // Every logit on the f32 MFMA, top-8 and quantisation in a launch of their own, from 240 tokens (where the grouping is a
+    // launch of its own as well). Whole layers against the chain router with both in its tail, us: 200 tokens 66.9 / 67.5,
+    // 333: 82.8 / 86.0, 511: 97.4 / 104.4. From 512 tokens only where exact logits are asked for: the default there is
+    // approximate logits on the bf16 MFMA with refinement, whose softmax sums differ by about 1e-7 (32-bit sums in another
+    // order), and what a size returns does not depend on which of the two is faster at it (512 97.5 / 101.5, 700 107.1 /
+    // 109.0, 1021 118.9 / 121.0, 1200 129.9 / 128.8).
+    if (order == MMOE_ORDER_BATCH && !w.norm_x && nb >= 240 && (nb < 512 || S_router_exact || exact_only))
         return launch(MMOE_K_ROUTER, [&] { kl(k_router_f32, dim3((nb + 15) / 16, MNE / (16 * RF_ET)), 512, 0, d_hn, nb, lw.rm, lw.bias, w.rl); });
     if (tk && nb < 512) {
         RouteTail rt{w.top, w.tw, w.qx, w.qsx, w.qsumx, hist, w.rcnt};
@@ -310,7 +312,8 @@ static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int or
     }
     // approximate logits on the bf16 MFMA; k_refine_topk makes the top-8 exact
     w.refine = true;
-    return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<8, 1>, dim3((nb + 31) / 32, MNE / 256, 4), 512, 0, lw.router, d_hn, nb, w.rpart); });
+    if (nb >= 1024) return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<8, 1>, dim3((nb + 31) / 32, MNE / 256, 4), 512, 0, lw.router, d_hn, nb, w.rpart); });
+    return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<4, 1>, dim3((nb + 31) / 32, MNE / 128, 4), 256, 0, lw.router, d_hn, nb, w.rpart); });
 }
 
 // the router launch, recording whether rl now holds every logit exactly (mmoe_route may then take them as they are)
@@ -318,8 +321,7 @@ static int stage_router(Work &w, int L, const float *d_hn, int nb, int order, bo
                         int *hist = nullptr) {
     w.rl_nb = 0;
     int rc = stage_router_launch(w, L, d_hn, nb, order, exact_only, tk, hist);
-    // (from 512 tokens mmoe_route takes them only from calls that ask for exact logits)
-    if (!rc && !w.refine && (order == MMOE_ORDER_STEP || nb < 512 || S_router_exact || exact_only)) w.rl_nb = nb;
+    if (!rc && !w.refine) w.rl_nb = nb;
     return rc;
 }
 

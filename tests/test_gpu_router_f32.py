@@ -1,7 +1,8 @@
 """The batch router on the f32 matrix cores (k_router_f32), which takes over at 240 tokens (384 in a stack), against the
 oracle's chains and against the chain router on the same tokens in smaller calls, bit for bit: the first sizes on either
-side of the switches, ragged token tiles of 16, and with exact logits asked for the sizes past 1023 up to the largest. And
-the approximate router with its refinement, for 1024 tokens and more, on logits that decide the top 8 by ties."""
+side of the switches, ragged token tiles of 16, and with exact logits asked for the sizes past 511 up to the largest. And
+the approximate router with its refinement, the default from 512 tokens: one token's results in batches of different sizes, and
+logits that decide the top 8 by ties."""
 import numpy as np
 import pytest
 
@@ -41,7 +42,7 @@ def test_router_f32_matches_chains(layer, nb, zipf):
     hn *= np.exp2(np.random.default_rng(nb).integers(-130, 40, size=(nb, 1))).astype(np.float32)
     hn[nb // 2] = 0
     hn = np.ascontiguousarray(hn)
-    M.check(lib.mmoe_set_router_mode(int(nb >= 1024)), "router mode")
+    M.check(lib.mmoe_set_router_mode(int(nb >= 512)), "router mode")
     try:
         rl, top, x = logits(hn)
         parts = [logits(np.ascontiguousarray(hn[i:i + 239])) for i in range(0, nb, 239)]
@@ -53,6 +54,19 @@ def test_router_f32_matches_chains(layer, nb, zipf):
     for b in (0, nb // 2, nb - 1):
         want = O.router_batch(hn[b:b + 1], layer.router, layer.bias if zipf else None)
         assert np.array_equal(rl[b:b + 1].view(np.int32), want.view(np.int32)), b
+
+
+@pytest.mark.parametrize("nb", [512, 700, 1023])
+def test_default_router_same_at_every_size(layer, nb):
+    """the default router from 512 tokens on gives a token the same logits and x whatever the size of its batch: the first
+    tokens of a batch of 1100, bit for bit (512 to 1023 tokens run blocks of 128 experts, from 1024 blocks of all 256)"""
+    lib = M.lib()
+    M.check(lib.mmoe_set_bias(L, M.ptr(layer.bias)), "bias")
+    _, hn = normed_hidden(SEED, 5650, 1100)
+    want = logits(hn)
+    got = logits(np.ascontiguousarray(hn[:nb]))
+    for a, b in zip(got, want):
+        assert np.array_equal(a.view(np.int32), b[:nb].view(np.int32))
 
 
 @pytest.mark.parametrize("nb", [383, 384])
