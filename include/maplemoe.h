@@ -86,7 +86,8 @@ int mmoe_dense_reset(void);
  * x += o), then post-norm and the router: rl gets nb x 256 logits; synchronous, returns device seconds (-1.0 on
  * error). gfull_moe adds the experts of the host's grouping into x (asynchronous). gfull_read waits, copies x
  * back and sets *ko to the chunk's fp16 k | v of every layer ([24][gfull_maxtok()][1024]; rows 0..nb-1 of each
- * layer are the chunk's, the rest are not refreshed). Results: k, v, x
+ * layer are the chunk's, the rest are not refreshed; *ko stays as it is until the next gfull_read that asks for ko, or
+ * gfull_init, also while later chunks run, and is another address each time). Results: k, v, x
  * after attention and the logits equal maple.c's CPU statements bit for bit. */
 int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t *router, const float *cs);
 void gfull_begin(const float *x, int nb, int pos0);

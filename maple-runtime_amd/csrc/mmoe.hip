@@ -769,9 +769,10 @@ static struct {
     float *cs;                    // [ctx][32][2]
     __half *kc; float *vc;        // [24][4 heads][sst][128] each: the fp16 cache values, v widened (attn.h)
     __half *ko;                   // [24][maxtok][1024]
-    uint16_t *ko_host;            // gfull_read's copy (pinned)
+    uint16_t *ko_host[2];         // keys and values on the host (pinned): ko_w is the block being filled, the other one is
+    int ko_w;                     // what gfull_read handed out last, which a caller may read while the next chunk runs
     hipEvent_t kev[24], cev;      // layer's keys and values written; copies so far done
-    uint32_t copied, busy;        // layers whose keys and values are on their way to ko_host (this chunk's; any chunk's)
+    uint32_t copied, busy;        // layers whose keys and values are on their way to ko_host[ko_w] (this chunk's; any chunk's)
     bool want_ko, captured;       // the last gfull_read asked for them; a caller has captured mmoe_gfull_stack
     float *qkv, *att, *sc, *inv, *mx;  // [maxtok][3072], [maxtok][2048], [maxtok * 16][ctx], [maxtok * 16] x 2
     double t_attn;
@@ -789,7 +790,7 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
                      (void **)&GF.qkv, (void **)&GF.att, (void **)&GF.sc, (void **)&GF.inv, (void **)&GF.mx};
     for (void **pp : dbuf) if (*pp) { HC(hipFree(*pp)); *pp = nullptr; }
     HC(hipStreamSynchronize(S.cst));
-    if (GF.ko_host) { HC(hipHostFree(GF.ko_host)); GF.ko_host = nullptr; }
+    for (uint16_t *&h : GF.ko_host) if (h) { HC(hipHostFree(h)); h = nullptr; }
     std::vector<uint16_t> nw((size_t)24 * GF_NWL);
     for (size_t i = 0; i < nw.size(); i++) { uint32_t u; memcpy(&u, &norms[i], 4); nw[i] = (uint16_t)(u >> 16); }
     HC(hipMalloc(&GF.nw, nw.size() * 2)); HC(hipMemcpy(GF.nw, nw.data(), nw.size() * 2, hipMemcpyHostToDevice));
@@ -798,12 +799,12 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     size_t kvb = (size_t)24 * GF.sst * 512 * 2, kob = (size_t)24 * maxtok * 1024 * 2;
     HC(hipMalloc(&GF.kc, kvb)); HC(hipMalloc(&GF.vc, 2 * kvb)); HC(hipMalloc(&GF.ko, kob));
     HC(hipMemset(GF.kc, 0, kvb)); HC(hipMemset(GF.vc, 0, 2 * kvb));
-    HC(hipHostMalloc((void **)&GF.ko_host, kob));
+    for (uint16_t *&h : GF.ko_host) HC(hipHostMalloc((void **)&h, kob));
     if (!GF.cev) {
         HC(hipEventCreateWithFlags(&GF.cev, hipEventDisableTiming));
         for (hipEvent_t &e : GF.kev) HC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    GF.copied = GF.busy = 0; GF.want_ko = true; GF.captured = false;
+    GF.ko_w = 0; GF.copied = GF.busy = 0; GF.want_ko = true; GF.captured = false;
     HC(hipMalloc(&GF.qkv, (size_t)maxtok * 3072 * 4)); HC(hipMalloc(&GF.att, (size_t)maxtok * MH * 4));
     HC(hipMalloc(&GF.sc, (size_t)maxtok * 16 * GF.sst * 4)); HC(hipMalloc(&GF.inv, (size_t)maxtok * 16 * 4)); HC(hipMalloc(&GF.mx, (size_t)maxtok * 16 * 4));
     for (int L = 0; L < 24; L++) {
@@ -819,10 +820,10 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
 }
 // a new chunk: nb hidden vectors (embeddings) at positions pos0..
 void gfull_begin(const float *x, int nb, int pos0) {
-    S.gfull_nb = 0;   // a rejected chunk leaves no chunk: gfull_attn / gfull_moe then report it
+    S.gfull_nb = 0; GF.copied = 0;   // a rejected chunk leaves no chunk: gfull_attn / gfull_moe then report it
     if (!S.gfull || nb < 1 || nb > S.main.maxtok) { seterr("gfull_begin: not set up or nb %d out of range", nb); return; }
     if (GF.ready && (nb > GF.maxtok || pos0 < 0 || pos0 + nb > GF.ctx)) { seterr("gfull_begin: positions %d..%d past ctx %d", pos0, pos0 + nb - 1, GF.ctx); return; }
-    S.gfull_nb = nb; GF.pos0 = pos0; GF.copied = 0;
+    S.gfull_nb = nb; GF.pos0 = pos0;
     HCV(hipMemcpyAsync(S.main.x, x, (size_t)nb * MH * 4, hipMemcpyHostToDevice, S.st));
 }
 // The attention half of layer L (asynchronous): x += o(attention(q, k, v of rmsnorm(x, in_ln))), k and v into
@@ -896,7 +897,7 @@ void gfull_moe(int nu, const uint32_t *loc, const int *regs, const int *ustart, 
     stage_combine(S.main, S.gfull_nb, S.main.x, MMOE_COMBINE_ADD);
 }
 // gpu_pre.m:569-584: waits, copies the hidden state back; *ko -> the chunk's k,v of every layer
-// (24 x maxtok x 1024 fp16, k | v per token; NULL before gfull_init)
+// (24 x maxtok x 1024 fp16, k | v per token; NULL before gfull_init), valid until the next call that asks for them
 void gfull_read(float *x, const uint16_t **ko) {
     HCV(hipStreamSynchronize(S.st));
     if (x && S.gfull) HCV(hipMemcpy(x, S.main.x, (size_t)S.gfull_nb * MH * 4, hipMemcpyDeviceToHost));
@@ -905,13 +906,15 @@ void gfull_read(float *x, const uint16_t **ko) {
         if (GF.ready) {   // the chunk's nb rows of every layer only (the [24][maxtok][1024] layout is kept)
             size_t pitch = (size_t)GF.maxtok * 1024 * 2, rows = (size_t)(S.gfull_nb ? S.gfull_nb : GF.maxtok) * 1024 * 2;
             HCV(hipStreamSynchronize(S.cst));
+            char *h = (char *)GF.ko_host[GF.ko_w];
             for (int L = 0, n; L < 24; L += n) {   // runs of layers that mmoe_gfull_stack has not copied beside its work
                 bool have = GF.copied >> L & 1;
                 for (n = 1; L + n < 24 && (GF.copied >> (L + n) & 1) == have; n++) {}
-                if (!have) HCV(hipMemcpy2D((char *)GF.ko_host + L * pitch, pitch, (char *)GF.ko + L * pitch, pitch, rows, n, hipMemcpyDeviceToHost));
+                if (!have) HCV(hipMemcpy2D(h + L * pitch, pitch, (char *)GF.ko + L * pitch, pitch, rows, n, hipMemcpyDeviceToHost));
             }
             GF.copied = GF.busy = 0;
-            *ko = GF.ko_host;
+            *ko = GF.ko_host[GF.ko_w];
+            GF.ko_w ^= 1;
         }
     }
     GF.want_ko = ko != nullptr;
@@ -1163,7 +1166,7 @@ static int ko_copy(int L) {
     size_t pitch = (size_t)GF.maxtok * 1024 * 2;
     HC(hipEventRecord(GF.kev[L], S.st));
     HC(hipStreamWaitEvent(S.cst, GF.kev[L], 0));
-    HC(hipMemcpyAsync((char *)GF.ko_host + L * pitch, (char *)GF.ko + L * pitch, (size_t)S.gfull_nb * 1024 * 2, hipMemcpyDeviceToHost, S.cst));
+    HC(hipMemcpyAsync((char *)GF.ko_host[GF.ko_w] + L * pitch, (char *)GF.ko + L * pitch, (size_t)S.gfull_nb * 1024 * 2, hipMemcpyDeviceToHost, S.cst));
     HC(hipEventRecord(GF.cev, S.cst));
     GF.copied |= 1u << L; GF.busy |= 1u << L;
     return 0;

@@ -1,7 +1,8 @@
 """Host data through the library's pinned blocks: gfull_moe calls queued one after the other (more than the ring of table
 blocks holds) against the same calls with a wait after each; and the keys and values that gfull_read hands out when
 mmoe_gfull_stack has copied them beside its work, against the ones gfull_read copies itself, over two chunks of
-different size, a chunk whose copies nobody read, a repeated stack and a partial one."""
+different size, a chunk whose copies nobody read, a repeated stack and a partial one, and the ones of a chunk left where
+they were handed out while the next chunk runs."""
 import ctypes as C
 
 import numpy as np
@@ -50,11 +51,16 @@ def test_queued_groupings(model):
     assert np.array_equal(out[0].view(np.int32), out[1].view(np.int32)) and not np.array_equal(out[0], x0)
 
 
-def read_kv(lib, nb):
+def held_kv(lib, nb):
+    """the chunk's keys and values where gfull_read hands them out"""
     p = C.c_void_p()
     lib.gfull_read(None, C.addressof(p))
     a = np.ctypeslib.as_array((C.c_uint16 * (24 * MAXTOK * 1024)).from_address(p.value)).reshape(24, MAXTOK, 1024)
-    return a[:NL, :nb].copy()
+    return a[:NL, :nb]
+
+
+def read_kv(lib, nb):
+    return held_kv(lib, nb).copy()
 
 
 def test_kv_copied_beside_the_stack(model):
@@ -95,6 +101,37 @@ def test_kv_copied_beside_the_stack(model):
     lib.gfull_begin(M.ptr(xs[0]), 200, 0)
     M.check(lib.mmoe_gfull_stack(0, NL), "stack"); M.check(lib.mmoe_gfull_stack(0, NL), "stack")
     assert np.array_equal(twice, read_kv(lib, 200)) and not np.array_equal(twice, want[0])
+
+
+def test_kv_held_over_the_next_chunks(model):
+    """what gfull_read handed out stays as it is until the next gfull_read that asks for it: over the next chunk's stack, over
+    further chunks that nobody reads, over a read of the hidden state alone, and over a rejected chunk"""
+    lib, _ = model
+    wait = C.CDLL("libamdhip64.so").hipDeviceSynchronize   # for the copies too
+    rng = np.random.default_rng(SEED + 82)
+    xs = [rng.standard_normal((nb, H)).astype(np.float32) for nb in (200, 56, 200, 200)]
+    pos, held, kept = 0, None, None
+
+    def chunk(x):
+        lib.gfull_begin(M.ptr(x), len(x), pos)
+        M.check(lib.mmoe_gfull_stack(0, NL), "stack")
+
+    for x in xs + xs[:2]:
+        pos = 0 if pos + len(x) > CTX else pos
+        chunk(x)
+        if held is not None:
+            assert wait() == 0 and np.array_equal(held, kept)
+            chunk(x)                                  # once more, unread
+            lib.gfull_begin(M.ptr(x), 0, pos)         # rejected
+            assert wait() == 0 and np.array_equal(held, kept)
+            chunk(x)
+            lib.gfull_read(None, None)
+            assert np.array_equal(held, kept)
+        now = held_kv(lib, len(x))
+        assert held is None or np.array_equal(held, kept)
+        held, kept = now, now.copy()
+        assert kept.any()
+        pos += len(x)
 
 
 @pytest.mark.parametrize("nb", [3, 8, 9])
