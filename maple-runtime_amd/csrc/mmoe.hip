@@ -1177,8 +1177,11 @@ int mmoe_gfull_stack(int L0, int nl) {
     if (L0 < 0 || nl < 1 || L0 + nl > 24) { seterr("mmoe_gfull_stack: layers %d..%d outside 0..23", L0, L0 + nl - 1); return -1; }
     if (!GF.ready || !S.gfull_nb) { seterr("mmoe_gfull_stack: gfull_init / gfull_begin first"); return -1; }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(S.st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipStreamSynchronize(S.cst);
+    HC(hipStreamIsCapturing(S.st, &cs));
+    if (cs != hipStreamCaptureStatusNone) {
+        // A replay writes the keys and values at any later time, without a wait for copies: from now on gfull_read makes them
+        // all. What copies that are under way bring is not used (gfull_read waits for them and copies again), so nothing
+        // has to wait for them here, where a capture would refuse or be broken by it.
         GF.captured = true; GF.copied = GF.busy = 0;
     }
     for (int L = L0; L < L0 + nl; L++) {

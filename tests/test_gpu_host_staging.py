@@ -1,8 +1,8 @@
 """Host data through the library's pinned blocks: gfull_moe calls queued one after the other (more than the ring of table
 blocks holds) against the same calls with a wait after each; and the keys and values that gfull_read hands out when
 mmoe_gfull_stack has copied them beside its work, against the ones gfull_read copies itself, over two chunks of
-different size, a chunk whose copies nobody read, a repeated stack and a partial one, and the ones of a chunk left where
-they were handed out while the next chunk runs."""
+different size, a chunk whose copies nobody read, a repeated stack and a partial one, the ones of a chunk left where they
+were handed out while the next chunk runs, and a stack that its caller captures and replays."""
 import ctypes as C
 
 import numpy as np
@@ -187,6 +187,48 @@ def test_grouping_under_capture(model, nb):
                 call(k)
             assert hip.hipGraphLaunch(ex, stream) == 0
             assert np.array_equal(read().view(np.int32), want.view(np.int32))
+    finally:
+        M.check(lib.mmoe_sync(), "sync")
+        hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("mode", [0, 1])   # global, thread-local
+@pytest.mark.parametrize("nb", [5, 200])
+def test_stack_under_capture(model, nb, mode):
+    """mmoe_gfull_stack captured by its caller while the copies of another chunk are under way, replayed with eager chunks in
+    between: hidden state, keys and values of every replay as the eager call's"""
+    lib, _ = model
+    hip = C.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(SEED + 95 + nb)
+    x0, x1 = (rng.standard_normal((n, H)).astype(np.float32) for n in (nb, 256))
+
+    def chunk(x, pos, stack):
+        lib.gfull_begin(M.ptr(x), len(x), pos)
+        stack()
+
+    def eager():
+        M.check(lib.mmoe_gfull_stack(0, NL), "stack")
+
+    def read():
+        x = np.empty((nb, H), np.float32)
+        lib.gfull_read(M.ptr(x), None)
+        return x.view(np.int32), read_kv(lib, nb)
+
+    chunk(x0, 0, eager)
+    want = read()
+    chunk(x1, 300, eager)
+    stream, graph, ex = C.c_void_p(lib.mmoe_stream()), C.c_void_p(), C.c_void_p()
+    lib.gfull_begin(M.ptr(x0), nb, 0)
+    assert hip.hipStreamBeginCapture(stream, mode) == 0
+    eager()
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    try:
+        for _ in range(3):
+            chunk(x0, 0, lambda: hip.hipGraphLaunch(ex, stream))
+            got = read()
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+            chunk(x1, 300, eager)
     finally:
         M.check(lib.mmoe_sync(), "sync")
         hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
