@@ -10,8 +10,9 @@
 //                 FMA chain over positions.
 // Work split: scores and the weighted sum of values run on the f32 matrix cores in tiles of 16 rows, 4 consecutive tokens
 // x the 4 query heads of one key/value head, so each cached key or value row is read once for the tile; a
-// token's own window is enforced with a zero weight outside it (an FMA with weight 0 leaves a chain unchanged,
-// exactly), so a tile shares one loop over positions.
+// token's own window is enforced with a zero weight outside it (an FMA with weight 0 and a finite value leaves a chain
+// unchanged, exactly), so a tile shares one loop over positions. Values past fp16's range are infinities in the cache: a
+// tile with such a position at the ends of its windows takes its tokens one by one (att_pv_tokens).
 #pragma once
 #include <hip/hip_fp16.h>
 #include "kernels.h"
@@ -44,11 +45,11 @@ __device__ __forceinline__ int att_kidx(int pos, int d) {
 // blocks, v widened to fp32: f32 MFMAs and vector instructions do not issue side by side on this part (a v_cvt_f32_f16
 // adds 5 cycles to a 33-cycle MFMA), and v has a conversion to an MFMA and a half. Keys widened as well cost more in bytes
 // than they save in conversions (k_att_scores at 2000 tokens, global layer: 134 us against 92; k_att_pv with v in fp16
-// 115 against 110).
+// 115 against 110). vinf[pos]: a byte per wave, set where one of the position's values is not finite.
 __global__ void __launch_bounds__(256) k_qkn(float *__restrict__ qkv, int pos0, int glob, const uint16_t *__restrict__ qn,
                                              const uint16_t *__restrict__ kn, const float *__restrict__ cs,
-                                             __half *__restrict__ kc, float *__restrict__ vc, __half *__restrict__ ko,
-                                             float *__restrict__ mx, int ctx) {
+                                             __half *__restrict__ kc, float *__restrict__ vc, uint32_t *__restrict__ vinf,
+                                             __half *__restrict__ ko, float *__restrict__ mx, int ctx) {
     __shared__ float xs[20 * AT_XS];
     __shared__ float kk[20];
     int b = blockIdx.x, t = threadIdx.x, pos = pos0 + b;
@@ -72,8 +73,11 @@ __global__ void __launch_bounds__(256) k_qkn(float *__restrict__ qkv, int pos0, 
         for (int m = 0; m < 2; m++) {
             int i = t + 256 * m;
             __half h = __float2half_rn(vv[m]);
-            vc[((size_t)(i >> 7) * ctx + pos) * AT_HD + (i & 127)] = __half2float(h); ko[(size_t)b * 1024 + 512 + i] = h;
+            vv[m] = __half2float(h);
+            vc[((size_t)(i >> 7) * ctx + pos) * AT_HD + (i & 127)] = vv[m]; ko[(size_t)b * 1024 + 512 + i] = h;
         }
+        bool bad = __ballot(!__builtin_isfinite(vv[0]) || !__builtin_isfinite(vv[1])) != 0;
+        if ((t & 63) == 0) ((uint8_t *)(vinf + pos))[t >> 6] = bad;
     }
     __syncthreads();
     if (t < 20) {
@@ -223,6 +227,31 @@ __device__ __forceinline__ void att_load_v(float2 *v, const float *vc, int blk, 
     for (int s = 0; s < 4; s++) v[s] = *(const float2 *)(base + (int32_t)lane_off + d[s]);
 }
 
+// Whether the tile's zero weights (positions that not every token sees, clamped ones, the block past an odd last one) meet a
+// value that is not finite. Uniform over the wave.
+__device__ __forceinline__ bool att_vinf(const uint32_t *vinf, const AttTile &T, int lane) {
+    int a = min(T.lo + lane, T.in0), b = min((T.in1 & ~15) + lane, T.hi);   // at most 4 and 19 positions
+    return __ballot((vinf[a] | vinf[b]) != 0) != 0;
+}
+// acc0 / acc1 += w (A operand, row = lane % 16) x the values of block blk as the tile's tokens see them: each token runs its
+// own products, with zeros for the values outside its window, and keeps the rows that are its own (lane (g, n) holds rows
+// 4 g + i: token g).
+__device__ __forceinline__ void att_pv_tokens(v4f &acc0, v4f &acc1, v4f w, const float2 *v, int blk, const AttTile &T, int glob, int win, int g) {
+#pragma unroll 1
+    for (int t = 0; t < AT_G; t++) {
+        v4f a0 = acc0, a1 = acc1;
+        int lo = att_lo(T.in1 + t, glob, win);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            int p = blk * 16 + 4 * s + g;
+            bool in = p >= lo && p <= T.in1 + t;
+            a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], in ? v[s].x : 0.0f, a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], in ? v[s].y : 0.0f, a1, 0, 0, 0);
+        }
+        if (g == t) { acc0 = a0; acc1 = a1; }
+    }
+}
+
 // The scores of a chunk whose windows are too long for k_att_local. One wave takes blocks of 16 positions w, w + 4, ... of
 // the workgroup's run (grid y; run: blocks per workgroup, a multiple of 4), the next block's keys loaded during the
 // current one's MFMAs. mx is raised to the row maxima. Bound: f32 MFMA issue (75 T FMA/s on registers) plus the
@@ -261,7 +290,7 @@ __global__ void __launch_bounds__(256, 3) k_att_scores(const float *__restrict__
 // per row (an even number of blocks and 4 more, so the 16 rows of a 16-byte read fall in different banks).
 __global__ void __launch_bounds__(256, 3) k_att_local(const float *__restrict__ qkv, int nb, int pos0, int glob, int win,
                                                       const __half *__restrict__ kc, const float *__restrict__ vc,
-                                                      float *__restrict__ att, int ldt, int sst) {
+                                                      const uint32_t *__restrict__ vinf, float *__restrict__ att, int ldt, int sst) {
     extern __shared__ __attribute__((aligned(16))) float att_s[];
     __shared__ float red[4][16], inv_s[16];
     int ntl = (nb + AT_G - 1) / AT_G, tile = ntl - 1 - (int)(blockIdx.x >> 2), kvh = blockIdx.x & 3;
@@ -299,6 +328,7 @@ __global__ void __launch_bounds__(256, 3) k_att_local(const float *__restrict__ 
     // the first values while the sums are added
     uint32_t lo_v = (uint32_t)(g * AT_HD + wv * 32 + 2 * n) * 4;
     float2 va[4], vb[4];
+    const bool vi = att_vinf(vinf, T, l);
     att_load_v(va, vc, bk0, T, lo_v, g);
     if (tid < 16) {   // in position order (4 words hold a block's positions 4 i + g)
         const float4 *q4 = (const float4 *)(att_s + tid * ldt);
@@ -323,9 +353,15 @@ __global__ void __launch_bounds__(256, 3) k_att_local(const float *__restrict__ 
             acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ws, v[s].y, acc1, 0, 0, 0);
         }
     };
-    // two blocks a turn (an odd last one is followed by a block of zero weights), each one's values loaded during the other's
-    // MFMAs
-    for (int k = 0; k < nblk; k += 2) {
+    if (__builtin_expect(vi, 0))
+        for (int k = 0; k < nblk; k++) {
+            v4f w = *(const v4f *)(wr + k * 16) * iv;
+            att_load_v(va, vc, bk0 + k, T, lo_v, g);
+            att_pv_tokens(acc0, acc1, w, va, bk0 + k, T, glob, win, g);
+        }
+    else for (int k = 0; k < nblk; k += 2) {
+        // two blocks a turn (an odd last one is followed by a block of zero weights), each one's values loaded during the
+        // other's MFMAs
         att_load_v(vb, vc, bk0 + min(k + 1, nblk - 1), T, lo_v, g);
         __builtin_amdgcn_sched_barrier(0);
         block(k, va);
@@ -405,7 +441,7 @@ __global__ void __launch_bounds__(256) k_att_softmax(int pos0, int glob, int win
 // their scores loaded one stage further ahead. Two row tiles per wave (a value row then feeds both) measured no faster.
 __global__ void __launch_bounds__(256) k_att_pv(int nb, int pos0, int glob, int win, const float *__restrict__ sc,
                                                 const float *__restrict__ mx, const float *__restrict__ inv, const float *__restrict__ vc,
-                                                float *__restrict__ att, int sst) {
+                                                const uint32_t *__restrict__ vinf, float *__restrict__ att, int sst) {
     constexpr int CH = 128, LD = CH + 4, PT = 16 * CH / 4 / 256;   // PT 16-byte words of scores per thread
     __shared__ __attribute__((aligned(16))) float wl[2][16 * LD];
     int ntl = (nb + AT_G - 1) / AT_G, tile = ntl - 1 - (int)(blockIdx.x >> 2), kvh = blockIdx.x & 3;
@@ -448,6 +484,21 @@ __global__ void __launch_bounds__(256) k_att_pv(int nb, int pos0, int glob, int 
             acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], v[s].y, acc1, 0, 0, 0);
         }
     };
+    const bool vi = att_vinf(vinf, T, l);
+    if (__builtin_expect(vi, 0)) {   // token by token, stage after stage; ahead of the loop below, whose registers it would add to
+        for (int p0 = c0; p0 < cend; p0 += CH) {
+            __syncthreads();
+            load(p0);
+            weights(p0, wl[0]);
+            __syncthreads();
+            for (int bk = p0 >> 4; bk < min(p0 + CH, cend) >> 4; bk++) {
+                att_load_v(va, vc, bk, T, lo_v, g);
+                att_pv_tokens(acc0, acc1, *(const v4f *)(wl[0] + n * LD + 4 * g + (bk * 16 - p0)), va, bk, T, glob, win, g);
+            }
+        }
+        __syncthreads();
+        cend = c0;   // nothing left for the loop below
+    }
     load(c0);
     att_load_v(va, vc, c0 >> 4, T, lo_v, g);
     weights(c0, wl[0]);

@@ -768,6 +768,7 @@ static struct {
     uint16_t *nw;                 // bf16 [24][4352] (the fp32 norms are bf16 values: exact)
     float *cs;                    // [ctx][32][2]
     __half *kc; float *vc;        // [24][4 heads][sst][128] each: the fp16 cache values, v widened (attn.h)
+    uint32_t *vinf;               // [24][sst]: positions with a value that is not finite (k_qkn)
     __half *ko;                   // [24][maxtok][1024]
     uint16_t *ko_host[2];         // keys and values on the host (pinned): ko_w is the block being filled, the other one is
     int ko_w;                     // what gfull_read handed out last, which a caller may read while the next chunk runs
@@ -786,7 +787,7 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     }
     // a second set-up replaces the first; buffers of a set-up that failed part way are released here too
     GF.ready = 0;
-    void **dbuf[] = {(void **)&GF.nw, (void **)&GF.cs, (void **)&GF.kc, (void **)&GF.vc, (void **)&GF.ko,
+    void **dbuf[] = {(void **)&GF.nw, (void **)&GF.cs, (void **)&GF.kc, (void **)&GF.vc, (void **)&GF.vinf, (void **)&GF.ko,
                      (void **)&GF.qkv, (void **)&GF.att, (void **)&GF.sc, (void **)&GF.inv, (void **)&GF.mx};
     for (void **pp : dbuf) if (*pp) { HC(hipFree(*pp)); *pp = nullptr; }
     HC(hipStreamSynchronize(S.cst));
@@ -799,6 +800,8 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
     size_t kvb = (size_t)24 * GF.sst * 512 * 2, kob = (size_t)24 * maxtok * 1024 * 2;
     HC(hipMalloc(&GF.kc, kvb)); HC(hipMalloc(&GF.vc, 2 * kvb)); HC(hipMalloc(&GF.ko, kob));
     HC(hipMemset(GF.kc, 0, kvb)); HC(hipMemset(GF.vc, 0, 2 * kvb));
+    size_t vib = (size_t)24 * GF.sst * 4;
+    HC(hipMalloc(&GF.vinf, vib)); HC(hipMemset(GF.vinf, 0, vib));
     for (uint16_t *&h : GF.ko_host) HC(hipHostMalloc((void **)&h, kob));
     if (!GF.cev) {
         HC(hipEventCreateWithFlags(&GF.cev, hipEventDisableTiming));
@@ -843,6 +846,7 @@ static int gfull_attn_launch(int L, int glob) {
     const uint16_t *nwl = GF.nw + (size_t)L * GF_NWL;
     __half *kcl = GF.kc + (size_t)L * sst * 512;
     float *vcl = GF.vc + (size_t)L * sst * 512;
+    uint32_t *vil = GF.vinf + (size_t)L * sst;
     __half *kol = GF.ko + (size_t)L * GF.maxtok * 1024;
     if (launch(MMOE_K_RMSNORM, [&] { kl(k_rmsnorm, nb, 256, 0, w.x, nwl, w.hn, nb); })) return -1;
     if (stage_quant_x(w, w.hn, nb)) return -1;
@@ -850,13 +854,13 @@ static int gfull_attn_launch(int L, int glob) {
         kl(k_dense<DENSE_W>, dim3(3072 / (64 * DENSE_W), (nb + 63) / 64), 64 * DENSE_W, 0, DN.dmat + g * 3, DN.drbs + g * 4, DN.n[g], nb, 3072, w.qx, w.qsx, w.qsumx, GF.qkv);
     })) return -1;
     if (launch(MMOE_K_QKN, [&] {
-        kl(k_qkn, nb, 256, 0, GF.qkv, pos0, glob, nwl + 4096, nwl + 4224, GF.cs, kcl, vcl, kol, GF.mx, sst);
+        kl(k_qkn, nb, 256, 0, GF.qkv, pos0, glob, nwl + 4096, nwl + 4224, GF.cs, kcl, vcl, vil, kol, GF.mx, sst);
     })) return -1;
     // blocks of 16 positions that a row tile's windows can overlap
     int tiles = (nb + AT_G - 1) / AT_G * 4, span = glob ? pos0 + nb : std::min(pos0 + nb, win + AT_G), blocks = (span + 15) / 16 + 1;
     if (blocks * 16 <= AT_LOCAL_T) {
         int ldt = (blocks + 1) / 2 * 32 + 4;
-        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_local, tiles, 256, (size_t)16 * ldt * 4, GF.qkv, nb, pos0, glob, win, kcl, vcl, GF.att, ldt, sst); })) return -1;
+        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_local, tiles, 256, (size_t)16 * ldt * 4, GF.qkv, nb, pos0, glob, win, kcl, vcl, vil, GF.att, ldt, sst); })) return -1;
     } else {
         // one run of k_att_scores takes a tile's whole window, unless the tiles alone are fewer than 1024 workgroups (then
         // runs of at least 8 blocks)
@@ -865,7 +869,7 @@ static int gfull_attn_launch(int L, int glob) {
             kl(k_att_scores, dim3(tiles, (blocks + run - 1) / run), 256, 0, GF.qkv, nb, pos0, glob, win, kcl, GF.sc, GF.mx, sst, run);
         })) return -1;
         if (launch(MMOE_K_ATT_SOFTMAX, [&] { kl(k_att_softmax, nb, 256, 0, pos0, glob, win, GF.sc, GF.mx, GF.inv, sst); })) return -1;
-        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_pv, tiles, 256, 0, nb, pos0, glob, win, GF.sc, GF.mx, GF.inv, vcl, GF.att, sst); })) return -1;
+        if (launch(MMOE_K_ATT_PV, [&] { kl(k_att_pv, tiles, 256, 0, nb, pos0, glob, win, GF.sc, GF.mx, GF.inv, vcl, vil, GF.att, sst); })) return -1;
     }
     if (stage_quant_x(w, GF.att, nb)) return -1;
     return launch(MMOE_K_DENSE, [&] {

@@ -34,3 +34,40 @@ def test_attn_tiles(gfull_model, nb, pos0):  # noqa: F811
         xo, ko_o, _ = O.attn_chunk(layers[L % 2], x0, pos0, glob, kc, vc, cs)
         assert np.array_equal(ko, ko_o), f"layer {L}: k/v"
         assert np.array_equal(x.view(np.uint32), xo.view(np.uint32)), f"layer {L}: x"
+
+
+@pytest.mark.parametrize("win,chunks", [(512, [(0, 8, 3)]), (512, [(600, 9, 2)]), (512, [(0, 8, 3), (512, 10, 7)]), (600, [(0, 7, 2), (601, 9, 5)])])
+def test_values_past_fp16(gfull_model, win, chunks):  # noqa: F811
+    """one token of a chunk (pos0, nb, token) has values past fp16's range, which the cache holds as infinities: the tokens that
+    do not see it, in its row tile before it and after it left the window, are the oracle's bit for bit; those that see it
+    come out as in the oracle (NaN). Both attention paths: one workgroup, and the separate kernels (global layers from 576
+    positions on; a window of 600)"""
+    lib, layers, _, _, _, norms, router_all = gfull_model
+    cs, c = O.rope_table(CTX), 77
+    norms, ln = norms.copy(), [al.in_ln.copy() for al in layers]
+    big = np.float32(2.0 ** 24)                       # norm weight of a column that only the token's hidden state has
+    norms[:, c] = big
+    rng = np.random.default_rng(SEED + 70 + win)
+    try:
+        for al in layers:
+            al.in_ln[c] = big.view(np.uint32) >> 16
+        M.check(lib.gfull_init(CTX, 64, win, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init")
+        cache = {L: (np.zeros((CTX, 512), np.uint16), np.zeros((CTX, 512), np.uint16)) for L, _ in LAYERS}
+        for pos0, nb, bad in chunks:
+            x0 = rng.standard_normal((nb, H)).astype(np.float32)
+            x0[:, c] = 0
+            x0[bad, c] = 1
+            lib.gfull_begin(M.ptr(x0), nb, pos0)
+            for L, glob in LAYERS:
+                lib.gfull_write_x(M.ptr(x0))
+                assert lib.gfull_attn(L, glob, None) >= 0, lib.mmoe_last_error()
+                x = np.empty((nb, H), np.float32)
+                lib.gfull_read(M.ptr(x), None)
+                xo, _, att = O.attn_chunk(layers[L % 2], x0, pos0, glob, *cache[L], cs, win)
+                assert not np.isfinite(att[bad]).all()
+                for b in range(nb):
+                    same = (x[b].view(np.uint32) == xo[b].view(np.uint32)) | (np.isnan(x[b]) & np.isnan(xo[b]))
+                    assert same.all(), f"pos0 {pos0} layer {L} token {b}: {int((~same).sum())} values differ"
+    finally:
+        for al, a in zip(layers, ln):
+            al.in_ln[:] = a
