@@ -7,7 +7,8 @@
 // quantised). What bounds each kernel: the dependent loads (routing, then codes) at a few experts, the code stream from
 // about a hundred. Measured against the one-workgroup kernel at the sizes where the choice between them changes: see
 // split_use in mmoe.hip.
-// Results are k_expert16's and the decode kernels' bit for bit: the same integer sums, the same fp32 sequence.
+// Results are the decode kernels' bit for bit, and k_expert16's for finite inputs: the same integer sums, the same fp32
+// sequence.
 #pragma once
 #include "kernels.h"
 
@@ -175,7 +176,8 @@ __global__ void __launch_bounds__(256, 4) k_gu_split(const Plan *__restrict__ pl
         float gv = (float)(ag[i] - qsum) * qs * sg[i];
         float uv = (float)(au[i] - qsum) * qs * su[i];
         float gg = gv < 7.0f ? gv : 7.0f;
-        o[i] = silu_le7(gg) * __builtin_amdgcn_fmed3f(uv, -7.0f, 7.0f);
+        // maple.c's clamp of a NaN too (infinite inputs): the NaN; v_med3_f32 would make it -7
+        o[i] = silu_le7(gg) * __builtin_elementwise_minimum(__builtin_elementwise_maximum(uv, -7.0f), 7.0f);
     }
     *(float4 *)(act + (size_t)(p0 + r16) * MFF + row0 + 4 * G) = make_float4(o[0], o[1], o[2], o[3]);
     if (dbg) {

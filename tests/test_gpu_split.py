@@ -54,6 +54,25 @@ def test_split_matches_three_kernels(layer, nb, order, zipf):
         M.check(lib.mmoe_set_expert_path(1), "expert path"); M.check(lib.mmoe_set_decode_path(1), "decode path")
 
 
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("nb", [2, 3, 8, 32])
+def test_split_infinite_inputs(layer, nb, order):
+    """tokens with infinite values beside ordinary ones: every token's x as from a call of its own (the one-token decode
+    kernels), bit for bit"""
+    lib = M.lib()
+    M.check(lib.mmoe_set_bias(L, None), "bias")
+    x, hn = normed_hidden(SEED, 5250 + nb, nb)
+    hn[0] = np.inf
+    hn[nb // 2, 100] = -np.inf
+    hn[-1, 2047] = np.inf
+    xg = x.copy()
+    M.check(lib.mmoe_moe(L, M.ptr(hn), nb, M.ptr(xg), order), "mmoe_moe")
+    for b in range(nb):
+        h, want = hn[b:b + 1].copy(), x[b:b + 1].copy()
+        M.check(lib.mmoe_moe(L, M.ptr(h), 1, M.ptr(want), order), "mmoe_moe")
+        assert ((xg[b].view(np.int32) == want[0].view(np.int32)) | (np.isnan(xg[b]) & np.isnan(want[0]))).all(), b
+
+
 @pytest.fixture(scope="module")
 def slots(layer):
     lib = M.lib()
