@@ -149,7 +149,7 @@ def test_gfull_whole_layers(gfull_model):
 def test_gfull_stack_on_device(gfull_model):
     """mmoe_gfull_stack: the attention half and the device MoE block (router, top-8, grouping, experts, combine)
     per layer with no host step between them. Layers 0..3 (3 is global) one at a time from the card's own input,
-    against the oracle's attention half followed by its MoE block; chunks of 5 tokens (the decode kernels) and
+    against the oracle's attention half followed by its MoE block; chunks of 5 tokens and
     of 256 tokens at positions past the window."""
     lib, layers, post, routers, cs = gfull_model[:5]
     blocks = [HostLayer(SEED, k) for k in range(2)]
@@ -182,20 +182,20 @@ def test_gfull_stack_on_device(gfull_model):
             assert e <= 1e-5
 
 
-@pytest.mark.parametrize("nb,pos0", [(1030, 0), (602, 700)])
-def test_gfull_attn_large_chunk(gfull_model, nb, pos0):
-    """Chunks of 1030 tokens at position 0 and 602 tokens at 700 (above 256 tokens the weighted-sum kernel takes
-    4-token groups; both sizes leave a partial group) on a fresh 2048-position set-up, local and global layer,
-    against the oracle."""
-    lib, layers, post, routers, cs, norms, router_all = gfull_model
+@pytest.mark.parametrize("nb,pos0,win,layers", [(1030, 0, O.WIN, LAYERS), (602, 700, O.WIN, LAYERS), (1030, 900, 600, LAYERS[:1])])
+def test_gfull_attn_large_chunk(gfull_model, nb, pos0, win, layers):
+    """Chunks of 1030 tokens at position 0 and 602 tokens at 700 (row tiles of 4 tokens; both sizes leave a partial
+    tile) on a fresh 2048-position set-up, local and global layer, and 1030 tokens with a window of 600 (the separate
+    score, softmax and weighted-sum kernels on a local layer), against the oracle."""
+    lib, mats, post, routers, cs, norms, router_all = gfull_model
     ctx = 2048
     cs = O.rope_table(ctx)
-    M.check(lib.gfull_init(ctx, 2048, O.WIN, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init 2048")
+    M.check(lib.gfull_init(ctx, 2048, win, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init 2048")
     rng = np.random.default_rng(SEED + 45 + nb)
     x0 = rng.standard_normal((nb, H)).astype(np.float32)
     lib.gfull_begin(M.ptr(x0), nb, pos0)
     assert not lib.mmoe_last_error().startswith(b"gfull_begin"), lib.mmoe_last_error()
-    for L, glob in LAYERS:
+    for L, glob in layers:
         print(f"\n  nb={nb} layer {L} glob={glob}", flush=True)
         lib.gfull_write_x(M.ptr(x0))
         rl = np.empty((nb, 256), np.float32)
@@ -205,7 +205,7 @@ def test_gfull_attn_large_chunk(gfull_model, nb, pos0):
         lib.gfull_read(M.ptr(x), C.addressof(kop))
         ko = np.ctypeslib.as_array((C.c_uint16 * (24 * 2048 * 1024)).from_address(kop.value)).reshape(24, 2048, 1024)[L, :nb]
         kc = np.zeros((ctx, 512), np.uint16); vc = np.zeros((ctx, 512), np.uint16)   # positions before pos0: zeros on both sides
-        xo, ko_o, _ = O.attn_chunk(layers[L % 2], x0, pos0, glob, kc, vc, cs)
+        xo, ko_o, _ = O.attn_chunk(mats[L % 2], x0, pos0, glob, kc, vc, cs, win)
         nx = int((x.view(np.uint32) != xo.view(np.uint32)).sum())
         print(f"  differing: k/v {int((ko != ko_o).sum())}, x {nx}", flush=True)
         assert np.array_equal(ko, ko_o) and nx == 0

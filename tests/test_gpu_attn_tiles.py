@@ -1,7 +1,8 @@
 """gfull_attn at the edges of its row tiles (4 tokens) and position blocks (16), against the oracle, bit for bit: chunks of 1 to
 33 tokens whose first and last positions fall on, before and after a block, windows just inside and just past the 576
 positions that one workgroup holds on chip (k_att_local; longer ones take the separate kernels), the window's own start
-inside a block, and a context length that is no multiple of 16. Positions before the chunk are zero on both sides."""
+inside a block, and a context length that is no multiple of 16. Positions before the chunk are zero on both sides, except
+where an earlier chunk is part of the case."""
 import ctypes as C
 
 import numpy as np
@@ -34,6 +35,26 @@ def test_attn_tiles(gfull_model, nb, pos0):  # noqa: F811
         xo, ko_o, _ = O.attn_chunk(layers[L % 2], x0, pos0, glob, kc, vc, cs)
         assert np.array_equal(ko, ko_o), f"layer {L}: k/v"
         assert np.array_equal(x.view(np.uint32), xo.view(np.uint32)), f"layer {L}: x"
+
+
+@pytest.mark.parametrize("win,nb,lo", [(600, 5, 16), (600, 9, 15), (600, 4, 17), (600, 33, 3), (777, 6, 30), (557, 13, 31)])
+def test_attn_window_start(gfull_model, win, nb, lo):  # noqa: F811
+    """local layers whose windows are too long for one workgroup (from 557 positions on; 39 to 50 blocks over several
+    workgroups): the first token's window starts at position lo, at, before and inside a block of 16, among the 24 positions
+    of an earlier chunk"""
+    lib, layers, _, _, _, norms, router_all = gfull_model
+    cs, L = O.rope_table(CTX), 0
+    M.check(lib.gfull_init(CTX, 64, win, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init")
+    rng = np.random.default_rng(SEED + 65 + win + nb)
+    kc = np.zeros((CTX, 512), np.uint16); vc = np.zeros((CTX, 512), np.uint16)
+    for pos0, n in ((max(lo - 10, 0), 24), (lo + win, nb)):
+        x0 = rng.standard_normal((n, H)).astype(np.float32)
+        lib.gfull_begin(M.ptr(x0), n, pos0)
+        assert lib.gfull_attn(L, 0, None) >= 0, lib.mmoe_last_error()
+        x = np.empty((n, H), np.float32)
+        lib.gfull_read(M.ptr(x), None)
+        xo, _, _ = O.attn_chunk(layers[L % 2], x0, pos0, 0, kc, vc, cs, win)
+        assert np.array_equal(x.view(np.uint32), xo.view(np.uint32)), f"chunk at {pos0}"
 
 
 @pytest.mark.parametrize("win,chunks", [(512, [(0, 8, 3)]), (512, [(600, 9, 2)]), (512, [(0, 8, 3), (512, 10, 7)]), (600, [(0, 7, 2), (601, 9, 5)])])

@@ -108,8 +108,8 @@ def test_silu_exhaustive():
 
 
 def test_moe_batch_gemm_router(layer0):
-    # >= 512 tokens with the exact router option: the tiled fp32 chains (k_router_gemm); 520 leaves a ragged
-    # last token tile
+    # >= 512 tokens with the exact router option: the chains on the f32 matrix cores (k_router_f32); 520 leaves a
+    # ragged last token tile
     M.check(M.lib().mmoe_set_router_mode(1), "router mode")
     try:
         compare_layer(layer0, 520, M.ORDER_BATCH)
@@ -117,28 +117,30 @@ def test_moe_batch_gemm_router(layer0):
         M.check(M.lib().mmoe_set_router_mode(0), "router mode")
 
 
-@pytest.mark.parametrize("nb,refined", [(255, False), (511, False), (512, True), (1023, True), (1024, True)])
+@pytest.mark.parametrize("nb,refined", [(239, False), (240, False), (255, False), (511, False), (512, True), (1023, True), (1024, True)])
 def test_moe_batch_size_boundaries(layer0, nb, refined):
-    """Sizes at the path switches: 255 tokens is the largest batch whose grouping forms inside the fused
-    small-tile kernel; 511 the last one on the chain router and 512 the first on the MFMA router with exact
+    """Sizes at the path switches: 239 tokens is the largest batch whose grouping forms inside the fused
+    small-tile kernel and the last one on the chain router, 240 the first on k_router_f32 and k_group (255: ragged
+    tiles of 16 tokens); 511 the last one with every logit exact and 512 the first on the MFMA router with exact
     refinement; 1023 runs the router in blocks of 128 experts (ragged last 32-token block), 1024 in blocks of
     all 256 experts."""
     compare_layer(layer0, nb, M.ORDER_BATCH, f" boundary {nb}", refined=refined)
 
 
 def test_moe_batch_tn64(layer0):
-    # 256 tokens -> 2048 pairs: the 64-token tile kernels
-    compare_layer(layer0, 256, M.ORDER_BATCH)
+    # from 360 tokens (2880 pairs) on the 64-pair tile kernels
+    compare_layer(layer0, 361, M.ORDER_BATCH)
+    assert M.read_plan()["tn"] == 64
 
 
 def test_moe_step(layer0):
     compare_layer(layer0, 1, M.ORDER_STEP)
 
 
-@pytest.mark.parametrize("nb", [48, 300])
-def test_gpre_moe(layer0, nb):
-    """gpre_moe with a host grouping (maple.c:757-763 call) vs the oracle's grouped experts; 300 tokens (2400
-    pairs) take the 64-pair tile kernels with a plan built from the host grouping"""
+@pytest.mark.parametrize("nb,tn", [(48, 16), (300, 16), (361, 64), (1000, 64)])
+def test_gpre_moe(layer0, nb, tn):
+    """gpre_moe with a host grouping (maple.c:757-763 call) vs the oracle's grouped experts; from 360 tokens (2880
+    pairs) on the 64-pair tile kernels run with a plan built from the host grouping"""
     lib = M.lib()
     x, hn = normed_hidden(SEED, 900, nb)
     rl = O.router_batch(hn, layer0.router)
@@ -152,6 +154,7 @@ def test_gpre_moe(layer0, nb):
     sec = lib.gpre_moe(M.ptr(hn), nb, nu, M.ptr(loc), M.ptr(regs), None, M.ptr(g["ustart"]), M.ptr(g["utok"]),
                        M.ptr(g["uw"]), M.ptr(tp), M.ptr(y))
     assert sec >= 0, lib.mmoe_last_error()
+    assert M.read_plan()["tn"] == tn
     import ctypes as C
     exu = (O.Expert * nu)(*[layer0.table[int(e)] for e in g["ue"]])
     yo = np.zeros_like(y)
@@ -203,7 +206,7 @@ def test_gpux(layer0):
 
 @pytest.mark.parametrize("nb", [1, 5, 8])
 def test_moe_grouped_path_small_batches(layer0, nb):
-    """the grouped-GEMM kernels at decode sizes (the default there is the three-kernel decode path)"""
+    """the grouped-GEMM kernels at decode sizes (one token takes the three-kernel decode path by default)"""
     M.check(M.lib().mmoe_set_decode_path(0), "decode off")
     try:
         compare_layer(layer0, nb, M.ORDER_BATCH)
@@ -350,9 +353,10 @@ def test_moe_batch_tn64_compact_sums(layer0):
     lib = M.lib()
     M.check(lib.mmoe_set_debug(0), "debug off")
     try:
-        nb = 256
+        nb = 361
         x, hn = normed_hidden(SEED, 77, nb)
         xg = run_gpu(layer0.L, hn, x, M.ORDER_BATCH)
+        assert M.read_plan()["tn"] == 64
         xo = x.copy()
         o = O.moe_batch(hn, layer0.router, layer0.table, xo)
         P = nb * 8
@@ -461,11 +465,12 @@ def test_combine_int16_overflow():
     M.check(lib.mmoe_set_bias(L, M.ptr(bias)), "bias")
     M.check(lib.mmoe_set_debug(0), "debug off")
     try:
-        nb = 256
+        nb = 361
         rng = np.random.default_rng(SEED + 5)
         hn = np.abs(rng.standard_normal((nb, 2048))).astype(np.float32)
         x = rng.standard_normal((nb, 2048)).astype(np.float32)
         xg = run_gpu(L, hn, x, M.ORDER_BATCH)
+        assert M.read_plan()["tn"] == 64   # the tiles whose down results travel as int16
         xo = x.copy()
         o = O.moe_batch(hn, router, O.experts_table(blk), xo, bias=bias, want=("top", "qa", "dn_i32"))
         assert (o["top"] == e).any(axis=1).all(), "every token routes to the all-ones expert"
@@ -545,10 +550,10 @@ def test_zipf_mfma_router_matches_exact(zipf_layer):
         M.check(lib.mmoe_set_debug(1), "debug on")
 
 
-@pytest.mark.parametrize("nb", [9, 100, 255])
+@pytest.mark.parametrize("nb", [9, 33, 100, 239, 255])
 def test_expert16_fused_matches_three_kernels(zipf_layer, nb):
-    """Tiles of 16 pairs: the fused whole-expert kernel (grouping, gate/up, act quantisation and down in one launch)
-    against k_group and the three separate kernels, bit for bit in every intermediate (the grouping's utok, uw,
+    """Tiles of 16 pairs: the fused kernels (33 to 239 tokens: grouping, gate/up, act quantisation and down in one launch;
+    9 and 255: gate/up and down over many workgroups) against k_group and the three separate kernels, bit for bit in every intermediate (the grouping's utok, uw,
     tp, sp and plan, int32 sums, act, its int8 quantisation, down) and in x. The Zipf bias gives experts of many tiles (the hot expert gets most tokens) next to single-pair
     tiles, so ragged tiles, padding rows and several workgroups per expert all occur."""
     lib = M.lib()
@@ -581,7 +586,7 @@ def test_expert16_fused_matches_three_kernels(zipf_layer, nb):
 
 @pytest.mark.parametrize("nb", [12, 40])
 def test_step_order_batch_matches_oracle(layer0, nb):
-    """A batch in step order above the decode path (the chain router's step order, the grouping inside the
+    """A batch in step order above one token (the chain router's step order, the grouping inside the
     small-tile kernel, the combine over slots sp/tw): every token's x equals maple.c's step() on that token alone,
     here the oracle's step restatement on sampled tokens, bit for bit in the top-8 and within the bar in x."""
     x, hn = normed_hidden(SEED, 4300 + nb, nb)

@@ -97,7 +97,7 @@ def route_dev(nb):
 @pytest.mark.parametrize("nb", [1, 300])
 def test_route_on_device_logits(ctx, nb):
     """rl = NULL: the routing of the logits a whole-layer call just computed on the device (the decode router at
-    one token, the chain router below 512 tokens), without a host copy; equal to the oracle's routing of those
+    one token, the f32 matrix-core router at 300), without a host copy; equal to the oracle's routing of those
     logits and to the layer call's own top-8."""
     from helpers import SEED, HostLayer, normed_hidden
     lib = M.lib()

@@ -1,8 +1,8 @@
 """mmoe_moe_dev_noalloc (work buffers in the library's static scratch, no allocation) against mmoe_moe_dev on
 the same inputs, bit for bit: two calls in a row, the second with a smaller batch, on the decode kernels
-(<= 8 tokens) and on the grouped 16-token-tile kernels (9..64 tokens), in both summation orders, and with the
-other kernel choices (the separate gate/up, quantisation and down kernels with k_group's per-chunk counts in the
-scratch; the grouped kernels for <= 8 tokens); sizes past the scratch are refused."""
+(one token), the split kernels (2 to 32 tokens) and the fused 16-pair-tile kernel (33 to 64), in both summation orders,
+and with the other kernel choices (the separate gate/up, quantisation and down kernels with k_group's per-chunk counts in
+the scratch; the grouped kernels for one token); sizes past the scratch are refused."""
 import numpy as np
 import pytest
 
