@@ -221,27 +221,22 @@ __device__ __forceinline__ float hsum8_lanes(float v) {
 // NORM: `in` is the hidden state x and the block first forms hn = rmsnorm(x, post_ln) for its token with
 // exactly k_rmsnorm's arithmetic (thread t sums columns t, t+256, ... in fp64, then the same 256-wide tree);
 // blocks with blockIdx.x == 0 write hn to hn_out. Else `in` is hn.
-// the top-8 / quantisation outputs of a router launch that also routes its tokens (TK); defined further down:
+// the top-8 / quantisation outputs of a router launch that also routes its tokens (k_router_chains2); defined further down:
 struct RouteTail { int *top; float *tw; int8_t *qx; float *qsx; int *qsumx; int *hist; int *cnt; };
 __device__ __forceinline__ int topk_wave(const float *__restrict__ r, float *E, int l, int *__restrict__ top, float *__restrict__ tw);
 
 template <int N, int GPAD = 0>
 __device__ __forceinline__ void quant_wave(const float *__restrict__ xr, int l, int8_t *__restrict__ q, float *__restrict__ qs,
                                            int *__restrict__ qsum);
-template <int NCH, bool NORM = false, bool TK = false>
-__global__ void __launch_bounds__(256) k_router_chains(const float *__restrict__ in, int nb, const uint16_t *__restrict__ wc,
+template <int NCH, bool NORM = false>
+__global__ void __launch_bounds__(256) k_router_chains(const float *__restrict__ in, const uint16_t *__restrict__ wc,
                                                        const float *__restrict__ bias, float *__restrict__ rl,
-                                                       const uint16_t *__restrict__ post_ln = nullptr, float *__restrict__ hn_out = nullptr,
-                                                       RouteTail tail = RouteTail{}) {
+                                                       const uint16_t *__restrict__ post_ln, float *__restrict__ hn_out) {
     constexpr int LEN = MH / NCH, HP = LEN + 4;
     __shared__ __attribute__((aligned(16))) float hc[NCH * HP];
     __shared__ double red[NORM ? 256 : 1];
     __shared__ float kk;
-    // TK: a 1-D grid in which the NCH blocks of token b (expert groups y) all get ids = b mod 8, i.e. run on
-    // XCD b mod 8 (workgroup ids go to the 8 XCDs round robin) and share its L2; else grid (NCH, nb)
-    int b = TK ? (int)(blockIdx.x / (8 * NCH)) * 8 + (int)(blockIdx.x % 8) : (int)blockIdx.y;
-    int y = TK ? (int)(blockIdx.x / 8) % NCH : (int)blockIdx.x;
-    if (TK && b >= nb) return;   // whole block
+    int b = blockIdx.y, y = blockIdx.x;   // token, expert group
     int tid = threadIdx.x, j = tid % NCH, e = y * (256 / NCH) + tid / NCH;
     const float *xr = in + (size_t)b * MH;
     float xv[8];
@@ -315,34 +310,12 @@ __global__ void __launch_bounds__(256) k_router_chains(const float *__restrict__
         if (bias) r = r + be;
         rl[(size_t)b * MNE + e] = r;
     }
-    if (TK) {
-        // the token's softmax/top-8 and int8 quantisation in the last of its NCH blocks to arrive: every block's
-        // stores (logits; hn from block 0) reach the XCD's L2 before its arrival is counted, and the last one
-        // reads them there (its L1 holds none of those lines: nothing in this kernel read them before)
-        __shared__ int last;
-        __shared__ __attribute__((aligned(16))) float E[MNE];
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid == 0) last = atomicAdd(&tail.cnt[b], 1) == NCH - 1;
-        __syncthreads();
-        if (!last) return;
-        int wv = tid >> 6, l = tid & 63;
-        if (wv == 0) {
-            int ek = topk_wave(rl + (size_t)b * MNE, E, l, tail.top + b * MTOPK, tail.tw + b * MTOPK);
-            if (tail.hist && l < MTOPK) atomicAdd(&tail.hist[(b >> 6) * MNE + ek], 1);   // per-chunk counts for k_group
-        } else if (wv == 1) {
-            const float *hr = (NORM ? hn_out : in) + (size_t)b * MH;
-            quant_wave<MH>(hr, l, tail.qx + (size_t)b * MH, tail.qsx + b, tail.qsumx + b);
-        } else if (tid == 128) {
-            tail.cnt[b] = 0;   // for the next launch (every block of the token has counted)
-        }
-    }
 }
 
-// k_router_chains for two tokens per block (the TK form: top-8 and quantisation in the last block): every thread
-// runs its chain for both tokens side by side from the same router words in registers, so a block reads its 32
-// experts' weights once for two tokens (half the blocks, half the L2 traffic) and the two FMA chains are
-// independent. Token pair q = (2q, 2q + 1) takes the NCH blocks with ids congruent to q mod 8 (one XCD). The
+// k_router_chains for two tokens per block, with their top-8 and quantisation: every thread runs its chain for both
+// tokens side by side from the same router words in registers, so a block reads its 32 experts' weights once for two
+// tokens (half the blocks, half the L2 traffic) and the two FMA chains are independent. Token pair q = (2q, 2q + 1)
+// takes the NCH blocks with ids congruent to q mod 8, i.e. one XCD (workgroup ids go to the 8 XCDs round robin). The
 // arithmetic per token is k_router_chains' exactly (the rmsnorm of each token as k_rmsnorm, the chains, the fold).
 template <int NCH, bool NORM>
 __global__ void __launch_bounds__(256) k_router_chains2(const float *__restrict__ in, int nb, const uint16_t *__restrict__ wc,
@@ -452,7 +425,9 @@ __global__ void __launch_bounds__(256) k_router_chains2(const float *__restrict_
         rl[(size_t)b0 * MNE + e] = r0;
         if (two) rl[(size_t)(b0 + 1) * MNE + e] = r1;
     }
-    // the pair's softmax/top-8 and quantisation in the last of its NCH blocks to arrive (as k_router_chains)
+    // the pair's softmax/top-8 and int8 quantisation in the last of its NCH blocks to arrive: every block's stores (logits;
+    // hn from the blocks y = 0) reach the XCD's L2 before its arrival is counted, and the last one reads them there (its
+    // L1 holds none of those lines: nothing in this kernel read them before)
     __shared__ int last;
     __shared__ __attribute__((aligned(16))) float E[2][MNE];
     __builtin_amdgcn_s_waitcnt(0);

@@ -257,15 +257,8 @@ static int tile_tn(int np) { return np >= (S_expert16 ? 2880 : 2048) ? 64 : 16; 
 
 // Router logits of nb tokens (d_hn) with layer L's router; order 0 = batch (maple.c:853-889), 1 = step (bf_row)
 static bool S_router_exact = false;   // batches of 512+: k_router_f32 (else MFMA logits + exact refinement)
-#ifndef ROUTER_TK
-#define ROUTER_TK 1
-#endif
-#ifndef ROUTER_TPB
-#define ROUTER_TPB 2   // tokens per block of the chain router with the top-8 tail (below 512 tokens)
-#endif
-static bool S_router_tk = ROUTER_TK;   // chain router: top-8 and quantisation in the router launch
 // exact_only: never the approximate large-batch router (callers that hand the logits themselves to the host)
-// tk (the chain router): the router launch also runs each token's softmax/top-8 (per-chunk counts into
+// tk (the chain router below 512 tokens): the router launch also runs each token's softmax/top-8 (per-chunk counts into
 // hist unless hist is null) and its int8 quantisation, in the last of the token's router blocks
 static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int order, bool exact_only, bool tk, int *hist) {
     LayerW &lw = S.layers[L];
@@ -285,31 +278,20 @@ static int stage_router_launch(Work &w, int L, const float *d_hn, int nb, int or
     if (tk && nb < 512) {
         RouteTail rt{w.top, w.tw, w.qx, w.qsx, w.qsumx, hist, w.rcnt};
         w.routed = true;
-        unsigned g8 = (unsigned)((nb + 7) / 8 * 8);
-        if (ROUTER_TPB == 2) {   // two tokens per block
-            unsigned p8 = (unsigned)(((nb + 1) / 2 + 7) / 8 * 8);
-            if (order == MMOE_ORDER_STEP) {
-                if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<16, true>, p8 * 16, 256, 0, w.norm_x, nb, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w, rt); });
-                return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<16, false>, p8 * 16, 256, 0, d_hn, nb, lw.rc16, lw.bias, w.rl, (const uint16_t *)nullptr, (float *)nullptr, rt); });
-            }
-            if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<8, true>, p8 * 8, 256, 0, w.norm_x, nb, lw.rc8, lw.bias, w.rl, w.norm_w, hn_w, rt); });
-            return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<8, false>, p8 * 8, 256, 0, d_hn, nb, lw.rc8, lw.bias, w.rl, (const uint16_t *)nullptr, (float *)nullptr, rt); });
-        }
+        unsigned p8 = (unsigned)(((nb + 1) / 2 + 7) / 8 * 8);
         if (order == MMOE_ORDER_STEP) {
-            if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16, true, true>, g8 * 16, 256, 0, w.norm_x, nb, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w, rt); });
-            return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16, false, true>, g8 * 16, 256, 0, d_hn, nb, lw.rc16, lw.bias, w.rl, nullptr, nullptr, rt); });
+            if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<16, true>, p8 * 16, 256, 0, w.norm_x, nb, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w, rt); });
+            return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<16, false>, p8 * 16, 256, 0, d_hn, nb, lw.rc16, lw.bias, w.rl, (const uint16_t *)nullptr, (float *)nullptr, rt); });
         }
-        if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8, true, true>, g8 * 8, 256, 0, w.norm_x, nb, lw.rc8, lw.bias, w.rl, w.norm_w, hn_w, rt); });
-        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8, false, true>, g8 * 8, 256, 0, d_hn, nb, lw.rc8, lw.bias, w.rl, nullptr, nullptr, rt); });
+        if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<8, true>, p8 * 8, 256, 0, w.norm_x, nb, lw.rc8, lw.bias, w.rl, w.norm_w, hn_w, rt); });
+        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains2<8, false>, p8 * 8, 256, 0, d_hn, nb, lw.rc8, lw.bias, w.rl, (const uint16_t *)nullptr, (float *)nullptr, rt); });
     }
     if (order == MMOE_ORDER_STEP) {
-        if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16, true>, dim3(MNE * 16 / 256, nb), 256, 0, w.norm_x, nb, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w, RouteTail{}); });
-        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16>, dim3(MNE * 16 / 256, nb), 256, 0, d_hn, nb, lw.rc16, lw.bias, w.rl, nullptr, nullptr, RouteTail{}); });
+        if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16, true>, dim3(MNE * 16 / 256, nb), 256, 0, w.norm_x, lw.rc16, lw.bias, w.rl, w.norm_w, hn_w); });
+        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<16>, dim3(MNE * 16 / 256, nb), 256, 0, d_hn, lw.rc16, lw.bias, w.rl, nullptr, nullptr); });
     }
-    if (nb < 240 || w.norm_x) {   // one block per (token, 32 experts): 8 nb blocks, router reread from L2 per token
-        if (w.norm_x) return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8, true>, dim3(MNE * 8 / 256, nb), 256, 0, w.norm_x, nb, lw.rc8, lw.bias, w.rl, w.norm_w, hn_w, RouteTail{}); });
-        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8>, dim3(MNE * 8 / 256, nb), 256, 0, d_hn, nb, lw.rc8, lw.bias, w.rl, nullptr, nullptr, RouteTail{}); });
-    }
+    if (nb < 240)   // one block per (token, 32 experts): 8 nb blocks, router reread from L2 per token
+        return launch(MMOE_K_ROUTER, [&] { kl(k_router_chains<8>, dim3(MNE * 8 / 256, nb), 256, 0, d_hn, lw.rc8, lw.bias, w.rl, nullptr, nullptr); });
     // approximate logits on the bf16 MFMA; k_refine_topk makes the top-8 exact
     w.refine = true;
     if (nb >= 1024) return launch(MMOE_K_ROUTER, [&] { kl(k_router_mfma<8, 1>, dim3((nb + 31) / 32, MNE / 256, 4), 512, 0, lw.router, d_hn, nb, w.rpart); });
@@ -481,7 +463,7 @@ static int moe_dev(Work &w, int L, const float *d_hn, int nb, float *d_x, int or
     // the chain router's launch also runs the top-8 and the quantisation; the per-chunk counts are for
     // k_group, which the fused small-tile kernel does without (it groups itself)
     bool grp16 = tn == 16 && S_expert16 && nb <= E16_GRP_MAXTOK;
-    if (stage_router(w, L, d_hn, nb, order, false, S_router_tk, grp16 ? nullptr : w.hist)) return -1;
+    if (stage_router(w, L, d_hn, nb, order, false, true, grp16 ? nullptr : w.hist)) return -1;
     int rc = stage_route_group(w, L, nb, tn, d_hn);
     // two or three tokens: the decode down kernel, which also combines (decode.h)
     if (!rc && nb <= DEC_MAXTOK && S_dec_enabled && w.grp16)
