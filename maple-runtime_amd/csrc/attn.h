@@ -119,13 +119,14 @@ __global__ void __launch_bounds__(256) k_qkn(float *__restrict__ qkv, int pos0, 
 // The score buffer: row (token b, head h) at (b * 16 + h) * sst, positions by their absolute index in blocks of 16, and
 // inside a block position 4 i + g at 4 g + i (g, i = 0..3): the 4 values that lane group g of k_att_pv's MFMAs multiplies in
 // its 4 steps are then one 16-byte word, and so are the 4 that a lane of k_att_scores' MFMAs holds. Every block that
-// overlaps the window of the row's 4-token group is written whole, -1e30 outside the token's own window: its exp is 0,
-// and a sum or an FMA chain is unchanged by a zero term, exactly.
+// overlaps the window of the row's 4-token group is written whole, -inf outside the token's own window: its exp is 0
+// whatever the row's maximum (at least -1e30, also where every score the token sees is -inf), and a sum or an FMA chain
+// is unchanged by a zero term, exactly.
 #define AT_G 4            // tokens per row tile: 4 tokens x 4 query heads = 16 MFMA rows
 #define AT_LOCAL_T 576    // longest window, in whole blocks, of k_att_local: 37 KB of scores, four workgroups per CU. With 1120
                           // (two per CU) a 1024-token chunk's layers take as long as with k_att_scores and the rest, with
                           // 2200 (one) a 2048-token chunk's 1.4 times as long
-// exp of x <= 0 (or -1e30): dexp without its overflow check
+// exp of x <= 0 (or -inf): dexp without its overflow check
 __device__ __forceinline__ float dexp_np(float x) {
     float k = __builtin_rintf(x * 1.44269504f);
     float r = __builtin_fmaf(-k, 0.693145752f, x);
@@ -194,7 +195,7 @@ __device__ __forceinline__ v4f att_score_block(const v4i *k, const AttRow &R, co
     }
     if (blk * 16 < T.in0 || blk * 16 + 15 > T.in1)   // uniform: some token does not see the whole block
 #pragma unroll
-        for (int i = 0; i < 4; i++) { int p = blk * 16 + 4 * i + g; o[i] = p >= R.lb && p <= R.pb ? o[i] : -1e30f; }
+        for (int i = 0; i < 4; i++) { int p = blk * 16 + 4 * i + g; o[i] = p >= R.lb && p <= R.pb ? o[i] : -__builtin_inff(); }
     return o;
 }
 // scores of blocks b, b + 4, ... below end: next(blk, o) for each; the next block's keys load during a block's MFMAs (past

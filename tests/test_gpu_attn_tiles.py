@@ -92,3 +92,34 @@ def test_values_past_fp16(gfull_model, win, chunks):  # noqa: F811
     finally:
         for al, a in zip(layers, ln):
             al.in_ln[:] = a
+
+
+@pytest.mark.parametrize("win,nb", [(512, 5), (600, 590)])
+def test_scores_all_negative_infinity(gfull_model, win, nb):  # noqa: F811
+    """keys with a dim past fp16's range: every score is infinite, and where all the scores a token sees are -inf its softmax
+    sum is 0 (the positions of its tile that it does not see add nothing), so the attention output is the oracle's NaN,
+    which the o projection's quantisation takes as 0. Both attention paths"""
+    lib, layers, _, _, _, norms, router_all = gfull_model
+    cs, c = O.rope_table(CTX), 100                    # past the dims that rope mixes
+    norms, kn = norms.copy(), [al.k_norm.copy() for al in layers]
+    big = np.float32(2.0 ** 60)
+    norms[:, 4224 + c] = big
+    x0 = np.random.default_rng(SEED + 75 + nb).standard_normal((nb, H)).astype(np.float32)
+    try:
+        for al in layers:
+            al.k_norm[c] = big.view(np.uint32) >> 16
+        M.check(lib.gfull_init(CTX, 640, win, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init")
+        lib.gfull_begin(M.ptr(x0), nb, 0)
+        for L, glob in LAYERS:
+            lib.gfull_write_x(M.ptr(x0))
+            assert lib.gfull_attn(L, glob, None) >= 0, lib.mmoe_last_error()
+            x = np.empty((nb, H), np.float32)
+            lib.gfull_read(M.ptr(x), None)
+            kc = np.zeros((CTX, 512), np.uint16); vc = np.zeros((CTX, 512), np.uint16)
+            xo, _, att = O.attn_chunk(layers[L % 2], x0, 0, glob, kc, vc, cs, win)
+            assert np.isnan(att[0]).all()
+            bad = np.flatnonzero((x.view(np.uint32) != xo.view(np.uint32)).any(1))
+            assert len(bad) == 0, f"layer {L}: tokens {bad[:8]}"
+    finally:
+        for al, a in zip(layers, kn):
+            al.k_norm[:] = a
