@@ -132,6 +132,7 @@ static struct {
     // gpux
     int gx_layers = 0, gx_slots = 0; uint8_t *gx_mem = nullptr;
     hipEvent_t gx_ev = nullptr; int gx_np = 0; uint8_t *gx_out = nullptr;   // gx_out: pinned, the call's outputs
+    bool gx_captured = false;   // a caller has captured gpux_begin: its replays don't record gx_ev
     // gfull
     bool gfull = false; int gfull_nb = 0;
     double t_moe = 0.0;
@@ -957,23 +958,26 @@ static void *gpux_start(int L, const float *x, int nb, int nu, const int *slots,
     S.gx_np = 0;
     if (experts_host_grouping(w, nb, nu, ep, pstart, ptok, NULL, NULL, x)) return NULL;
     HCN(hipMemcpyAsync(S.gx_out, w.down, (size_t)pstart[nu] * MH * 4, hipMemcpyDeviceToHost, S.st));   // beside the caller's own work
-    HCN(hipEventRecord(S.gx_ev, S.st));
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HCN(hipStreamIsCapturing(S.st, &cs));
+    if (cs != hipStreamCaptureStatusNone) S.gx_captured = true;
+    else HCN(hipEventRecord(S.gx_ev, S.st));
     S.gx_np = pstart[nu];
     return (void *)&S.gx_ev;
 }
 static void gpux_finish(void *h, float *out, int np) {
     if (h != (void *)&S.gx_ev) { seterr("gpux_end: unknown handle"); return; }
     if (np != S.gx_np) { seterr("gpux_end: %d outputs asked, %d computed", np, S.gx_np); return; }
-    HCV(hipEventSynchronize(S.gx_ev));
+    if (S.gx_captured) HCV(hipStreamSynchronize(S.st));   // the outputs may be a replay's
+    else HCV(hipEventSynchronize(S.gx_ev));
     memcpy(out, S.gx_out, (size_t)np * MH * 4);
 }
+// one pair per expert, all of token 0: kept, since a captured call's graph reads them when it runs
+static const struct GpuxRuns { int start[MNE + 1], tok[MNE] = {}; GpuxRuns() { for (int k = 0; k <= MNE; k++) start[k] = k; } } gpux_runs;
 // n hits of one token: outputs out[k][2048] = down of slot k's expert (unweighted), maple.c:628-642
 void *gpux_begin(int L, const float *x, int n, const int *slots) {
-    int ps[MNE + 1], pt[MNE];
     if (n < 1 || n > MNE) { seterr("gpux_begin: n %d", n); return NULL; }
-    for (int k = 0; k <= n; k++) ps[k] = k;
-    for (int k = 0; k < n; k++) pt[k] = 0;
-    return gpux_start(L, x, 1, n, slots, ps, pt);
+    return gpux_start(L, x, 1, n, slots, gpux_runs.start, gpux_runs.tok);
 }
 void gpux_end(void *h, float *out, int n) { gpux_finish(h, out, n); }
 void *gpux_begin_multi(int L, const float *x, int nb, int nu, const int *slots, const int *pstart, const int *ptok) {

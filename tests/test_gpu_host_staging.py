@@ -2,7 +2,7 @@
 blocks holds) against the same calls with a wait after each; and the keys and values that gfull_read hands out when
 mmoe_gfull_stack has copied them beside its work, against the ones gfull_read copies itself, over two chunks of
 different size, a chunk whose copies nobody read, a repeated stack and a partial one, the ones of a chunk left where they
-were handed out while the next chunk runs, and a stack that its caller captures and replays."""
+were handed out while the next chunk runs, and a stack and a gpux call that their caller captures and replays."""
 import ctypes as C
 
 import numpy as np
@@ -229,6 +229,45 @@ def test_stack_under_capture(model, nb, mode):
             got = read()
             assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
             chunk(x1, 300, eager)
+    finally:
+        M.check(lib.mmoe_sync(), "sync")
+        hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
+
+
+def test_gpux_under_capture(model):
+    """gpux_begin captured by its caller, replayed with other values in its input array and eager calls in between: gpux_end
+    after a replay gives the replay's outputs"""
+    lib, _ = model
+    hip = C.CDLL("libamdhip64.so")
+    M.check(lib.gpux_init(1, 8), "gpux_init")
+    hl = HostLayer(SEED, 0)
+    for s in range(8):
+        lib.gpux_upload(0, s, *[M.ptr(a) for a in M.expert_views(hl.blk, 11 * s)])
+    rng = np.random.default_rng(SEED + 99)
+    xs = rng.standard_normal((3, H)).astype(np.float32)
+    slots, few = np.arange(8, dtype=np.int32), np.array([5, 2], np.int32)
+
+    def end(h, n):
+        out = np.full((n, H), np.nan, np.float32)
+        lib.gpux_end(h, M.ptr(out), n)
+        return out.view(np.int32)
+
+    want = [end(lib.gpux_begin(0, M.ptr(x), 8, M.ptr(slots)), 8) for x in xs]
+    other = end(lib.gpux_begin(0, M.ptr(xs[0]), 2, M.ptr(few)), 2)
+    x = xs[0].copy()                                             # the captured call's input
+    stream, graph, ex = C.c_void_p(lib.mmoe_stream()), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    h = lib.gpux_begin(0, M.ptr(x), 8, M.ptr(slots))
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert h, lib.mmoe_last_error()
+    assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    try:
+        for k in (0, 1, 2, 1):
+            x[:] = xs[k]
+            assert hip.hipGraphLaunch(ex, stream) == 0
+            assert np.array_equal(end(h, 8), want[k]), f"replay {k}"
+            assert np.array_equal(end(lib.gpux_begin(0, M.ptr(xs[0]), 2, M.ptr(few)), 2), other)
+            assert np.array_equal(end(lib.gpux_begin(0, M.ptr(xs[0]), 8, M.ptr(slots)), 8), want[0])
     finally:
         M.check(lib.mmoe_sync(), "sync")
         hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
