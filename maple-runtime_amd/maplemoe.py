@@ -97,8 +97,12 @@ def _declare(L):
 
 
 def ptr(a):
-    """data pointer of a numpy array; the caller must keep the array referenced until the call returns"""
-    return None if a is None else C.c_void_p(a.ctypes.data)
+    """data pointer of a numpy array; it holds the array, so that a temporary lives until the call it is passed to returns"""
+    if a is None:
+        return None
+    p = C.c_void_p(a.ctypes.data)
+    p.array = a
+    return p
 
 
 def check(rc, what=""):

@@ -12,7 +12,12 @@ H, NE, TOPK, FF = 2048, 256, 8, 512
 
 
 def _p(a):
-    return None if a is None else C.c_void_p(a.ctypes.data)
+    """data pointer of a numpy array; it holds the array, so that a temporary lives until the call it is passed to returns"""
+    if a is None:
+        return None
+    p = C.c_void_p(a.ctypes.data)
+    p.array = a
+    return p
 
 
 class Expert(C.Structure):
