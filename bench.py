@@ -188,7 +188,7 @@ def cpu_baselines(blocks, routers, seconds):
     res = {}
     model, phys, usable = cpu_topology()
     # every core this process may use (the affinity mask), at most the host's physical cores (maple.c runs one
-    # thread per core) and at most the thread budget the environment sets (OMP_NUM_THREADS on the GPU boxes)
+    # thread per core) and at most the thread budget the environment sets (OMP_NUM_THREADS)
     budget = int(os.environ.get("OMP_NUM_THREADS", "0") or 0)
     nt_all = min(x for x in (usable, phys, budget or None) if x)
     for nt in (1, nt_all):

@@ -189,7 +189,7 @@ int mmoe_set_debug(int on);
 /* One token uses three fused decode kernels, two and three tokens their down kernel (default on); off = the grouped
  * path of larger batches. */
 int mmoe_set_decode_path(int on);
-/* Batches whose pairs are tiled by 16 (fewer than 2048 pairs, above the decode path): 1 (default) = the fused kernels
+/* Batches whose pairs are tiled by 16 (above the decode path; fewer than 2880 pairs, with 0 here 2048): 1 (default) = the fused kernels
  * (few experts: gate/up and down with the act quantisation, each expert over many workgroups; else one kernel per
  * tile), 0 = the three separate kernels. All give identical results. */
 int mmoe_set_expert_path(int fused);

@@ -70,7 +70,7 @@ struct Work {
     int *qsumx = nullptr, *qsuma = nullptr;
     int *dbg_gu = nullptr, *dbg_dn = nullptr;
     int *dov = nullptr;             // the same for the int16 down results
-    DnTile *dt = nullptr;           // tile records of the split down kernel [SP_MAXP]
+    DnTile *dt = nullptr;           // tile records of the split down kernel (as many as tiles)
     int *eu = nullptr, *pu = nullptr;   // expert -> used-expert index [256], pair -> used-expert index [P]
     bool compact = false;           // the last expert stage left down as int16 (k_combine16)
     int hist_used = 0;              // entries of hist the device grouping filled; the combine clears them
@@ -162,8 +162,8 @@ static void kl(void (*f)(P...), dim3 g, dim3 b, size_t shm, A &&...a) {
     if (e != hipSuccess) g_klerr = e;
 }
 
-// small (carved sets): at most 64 tokens, so only the decode and 16-token-tile paths run: no int16 down side
-// buffer (2048+ pairs only), no approximate-router buffers (512+ tokens), no host-side hidden state copy.
+// small (carved sets): at most 64 tokens, so only the decode and 16-pair-tile paths run: no int16 down side
+// buffer (tiles of 64 pairs only), no approximate-router buffers (512+ tokens), no host-side hidden state copy.
 static int work_alloc(Work &w, int maxtok, Carve *c = nullptr) {
     if (maxtok < 1 || maxtok > MMOE_MAXTOK || (c && maxtok > 64)) { seterr("maxtok %d outside 1..%d", maxtok, c ? 64 : MMOE_MAXTOK); return -1; }
     w.maxtok = maxtok; w.maxp = maxtok * MTOPK;

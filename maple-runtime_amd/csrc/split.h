@@ -2,10 +2,10 @@
 //
 // With few used experts, one workgroup per expert (k_expert16) leaves most CUs idle: a CU streams about 30 GB/s, so a
 // 798,720-byte expert takes 27 us however few there are. Here an expert's rows are split over 8 to 32 workgroups per
-// kernel, every wave issues all of its code loads at once (16 KB per gate/up wave, 8 KB per down wave), and act makes
-// one trip through HBM's caches between the two launches (every row of an expert is needed before its act can be
-// quantised). What bounds each kernel: the dependent loads (routing, then codes) at a few experts, the code stream from
-// about a hundred. Measured against the one-workgroup kernel at the sizes where the choice between them changes: see
+// kernel, every wave issues all of its code loads at once (16, 8 or 4 KB per gate/up wave for KS = 1, 2, 4; 4 KB per down
+// wave), and act makes one trip through HBM's caches between the two launches (every row of an expert is needed before
+// its act can be quantised). What bounds each kernel: the dependent loads (routing, then codes) at a few experts, the code
+// stream from about a hundred. Measured against the one-workgroup kernel at the sizes where the choice between them changes: see
 // split_use in mmoe.hip.
 // Results are the decode kernels' bit for bit, and k_expert16's for finite inputs: the same integer sums, the same fp32
 // sequence.

@@ -1,7 +1,7 @@
 """The drop-in boundary at build level: maple.c's own prototypes of its GPU entry points (maple.c:246-272,
 compiled with -DGPU_HEAD) agree with include/maplemoe.h in one translation unit, and the unchanged maple.c
 links against libmaplemoe.so with every GPU symbol resolved by it. Both read maple.c from /root/reference
-and are skipped where it is absent (the GPU box); nothing of maple.c is kept in the repository."""
+and are skipped where it is absent (machines without the reference); nothing of maple.c is kept in the repository."""
 import os
 import re
 import subprocess
