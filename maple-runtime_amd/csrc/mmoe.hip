@@ -487,11 +487,13 @@ static int experts_host_grouping(Work &w, int nb, int nu, const ExpPtr *eptr_h, 
     if (nu < 1 || nu > MNE) { seterr("nu %d outside 1..256", nu); return -1; }
     int np = ustart[nu];
     if (nb < 1 || nb > w.maxtok || np < 1 || np > w.maxp) { seterr("nb %d / pairs %d exceed capacity %d / %d", nb, np, w.maxtok, w.maxp); return -1; }
+    if (ustart[0] < 0) { seterr("ustart[0] = %d", ustart[0]); return -1; }
     for (int u = 0; u < nu; u++) if (ustart[u + 1] < ustart[u]) { seterr("ustart not ascending at %d", u); return -1; }
     for (int a = 0; a < np; a++) if (ptok[a] < 0 || ptok[a] >= nb) { seterr("ptok[%d] = %d outside 0..%d", a, ptok[a], nb - 1); return -1; }
     if (tp) for (int i = 0; i < nb * MTOPK; i++) if (tp[i] < 0 || tp[i] >= np) { seterr("tp[%d] = %d outside 0..%d", i, tp[i], np - 1); return -1; }
     int tn = tile_tn(np), ntile = 0;
     for (int u = 0; u < nu; u++) ntile += (ustart[u + 1] - ustart[u] + tn - 1) / tn;
+    ntile = std::max(ntile, 1);   // a grouping without pairs launches workgroups that find none
     HostGroup h{};
     h.nu = nu; h.np = np; h.ntp = tp ? nb * MTOPK : 0;
     const float *x = w.hn;

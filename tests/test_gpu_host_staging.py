@@ -271,3 +271,27 @@ def test_gpux_under_capture(model):
     finally:
         M.check(lib.mmoe_sync(), "sync")
         hip.hipGraphExecDestroy(ex); hip.hipGraphDestroy(graph)
+
+
+def test_grouping_without_pairs(model):
+    """a grouping whose experts have no pairs runs and changes nothing for the calls after it; one that starts below 0 is
+    refused"""
+    lib, _ = model
+    M.check(lib.gpux_init(1, 2), "gpux_init")
+    hl = HostLayer(SEED, 0)
+    for s in range(2):
+        lib.gpux_upload(0, s, *[M.ptr(a) for a in M.expert_views(hl.blk, s)])
+    x = np.random.default_rng(SEED + 98).standard_normal((2, H)).astype(np.float32)
+    slots, tok = np.array([0, 1], np.int32), np.zeros(2, np.int32)
+
+    def call(*start):
+        out, us = np.zeros((2, H), np.float32), np.array(start, np.int32)
+        h = lib.gpux_begin_multi(0, M.ptr(x), 2, 2, M.ptr(slots), M.ptr(us), M.ptr(tok))
+        if h:
+            lib.gpux_end_multi(h, M.ptr(out), 2)
+        return out if h else None
+
+    want = call(0, 1, 2)
+    assert want.any() and call(2, 2, 2) is not None
+    assert call(-1, 1, 2) is None and b"ustart[0]" in lib.mmoe_last_error()
+    assert np.array_equal(call(0, 1, 2).view(np.int32), want.view(np.int32))
