@@ -801,6 +801,7 @@ int gfull_init(int ctx, int maxtok, int win, const float *norms, const uint16_t 
         if (!lw.post_ln) HC(hipMalloc(&lw.post_ln, MH * 2));
         HC(hipMemcpy(lw.post_ln, nw.data() + (size_t)L * GF_NWL + MH, MH * 2, hipMemcpyHostToDevice));
     }
+    if (S.gfull_nb > maxtok || GF.pos0 + S.gfull_nb > ctx) S.gfull_nb = 0;   // a chunk begun before that the new buffers don't hold
     GF.ctx = ctx; GF.win = win; GF.maxtok = maxtok; GF.ready = 1;
     S.gfull = true;
     fprintf(stderr, "maplemoe: whole layers on the card, key/value cache %.0f MB\n", 3.0 * kvb / 1e6);

@@ -295,3 +295,24 @@ def test_grouping_without_pairs(model):
     assert want.any() and call(2, 2, 2) is not None
     assert call(-1, 1, 2) is None and b"ustart[0]" in lib.mmoe_last_error()
     assert np.array_equal(call(0, 1, 2).view(np.int32), want.view(np.int32))
+
+
+def test_smaller_setup_drops_the_chunk(model, gfull_model):  # noqa: F811
+    """a chunk begun under a larger set-up is no chunk of a smaller one: the calls that would use it say so"""
+    lib, _ = model
+    _, _, _, _, cs, norms, router_all = gfull_model
+    x = np.random.default_rng(SEED + 97).standard_normal((200, H)).astype(np.float32)
+
+    def init(ctx, maxtok):
+        M.check(lib.gfull_init(ctx, maxtok, O.WIN, M.ptr(norms), M.ptr(router_all), M.ptr(cs)), "gfull_init")
+
+    try:
+        for nb, pos, ctx, maxtok in ((200, 0, CTX, 64), (20, 300, 256, 64)):
+            init(CTX, MAXTOK)
+            lib.gfull_begin(M.ptr(x), nb, pos)
+            init(ctx, maxtok)
+            assert lib.gfull_attn(0, 0, None) < 0 and lib.mmoe_gfull_stack(0, 1) != 0
+            lib.gfull_begin(M.ptr(x), 20, 0)
+            assert lib.gfull_attn(0, 0, None) >= 0, lib.mmoe_last_error()
+    finally:
+        init(CTX, MAXTOK)
