@@ -1,7 +1,7 @@
 /* moe_oracle.c -- CPU restatement of maple-runtime's MoE hot path, for checking only.
  *
  * TEST INFRASTRUCTURE: loaded by tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg as the
- * checker. Never linked into the product. Build: oracle/Makefile (gcc -O2 -ffp-contract=off, no fast-math).
+ * oracle. Never linked into the product. Build: oracle/Makefile (gcc -O2 -ffp-contract=off, no fast-math).
  * See moe_oracle.h for the reference citation of every function and how each one is pinned.
  */
 #include "moe_oracle.h"

@@ -1,7 +1,7 @@
 /* moe_oracle.h -- CPU restatement of maple-runtime's MoE hot path, for checking only.
  *
  * TEST INFRASTRUCTURE. Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may load
- * this code, and only as the checker. The product library (libmaplemoe) never links or calls it.
+ * this code, and only as the oracle. The product library (libmaplemoe) never links or calls it.
  *
  * Every function follows a function or block of maple.c (the reference's C runtime); the citation is on
  * each declaration. Arithmetic is plain IEEE fp32/fp64 with no fast-math and no FMA contraction

@@ -1,4 +1,4 @@
-"""ctypes bindings of the checker: liboracle.so (the C restatement) and _ref/libmaple_ref.so (maple.c itself).
+"""ctypes bindings of the oracle: liboracle.so (the C restatement) and _ref/libmaple_ref.so (maple.c itself).
 
 TEST INFRASTRUCTURE: imported only by tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg.
 """
