@@ -1884,7 +1884,10 @@ __global__ void __launch_bounds__(WAVES * 64) k_down(const Plan *__restrict__ pl
 // utok, uw, sp, pu and tp (a pair's rank among its token's 8 pairs is the number of the token's experts with a
 // smaller id, since pairs are ordered by expert); workgroup 0 writes the plan, tile table, expert pointers and
 // eu as k_group does. The outputs equal k_group's.
-#define E16_GRP_MAXTOK 239   // 255 tokens: 86.8 us per layer (some CUs get a second tile) against 80 with k_group and the split kernels; 216: 68.7 / 76
+// The last size whose grouping k_expert16 forms; above it k_group and the split kernels. Whole layer, here / there, us:
+// 216 tokens, balanced experts 68.7 / 76; 240 tokens 75.0 / 76.9, with the Zipf bias 59.2 / 57.4; 253 tokens, when some
+// CUs get a second tile, 83.4 / 77.4 and 66.8 / 57.2.
+#define E16_GRP_MAXTOK 239
 struct GroupIn { const int *top; const float *tw; int nb; const ExpPtr *layer_tab; Plan *plan; Tile *tiles; ExpPtr *eptr_u;
                  int *eu; int *utok; float *uw; int *tp; int *sp; int *pu; };
 template <int WAVES, int RING, int GRP = 0, int GL = 8>
